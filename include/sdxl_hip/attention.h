@@ -49,8 +49,9 @@ typedef enum sdxl_dtype {
  *   WARP_ONLINE runs the wave64 online-softmax kernel (the reference's
  *     correctness fallback, any head_dim <= 1024, f16/bf16/f32);
  *   AUTO picks the fused kernel whenever it is eligible, else WARP_ONLINE,
- *     whose unmasked non-causal FP32 calls at head_dim 512 (the VAE) run a
- *     tiled fp32 matrix-core kernel instead of the per-row one. */
+ *     whose calls run tiled matrix-core kernels of fp32 accuracy instead of
+ *     the per-row one where they take the shape (head_dim <= 160; unmasked
+ *     non-causal FP32 at head_dim 512, the VAE). */
 typedef enum sdxl_attn_backend {
     SDXL_ATTN_AUTO = 0,
     SDXL_ATTN_CUDNN_SDPA = 1,
@@ -106,9 +107,9 @@ sdxl_status sdxl_attn_backend_parse(const char* name, int32_t* backend);
 const char* sdxl_attn_backend_name(int32_t backend);
 
 /* Name of the kernel family a resolved backend runs on this device:
- * "flash-gfx950" or "wave-online". Under the auto backend, unmasked non-causal
- * FP32 calls at head_dim 512 (the VAE's attention) resolve to the online
- * family but run its fp32 matrix-core kernel. */
+ * "flash-gfx950" or "wave-online". Under the auto backend, calls of the online
+ * family at head_dim <= 160 and unmasked non-causal FP32 calls at head_dim 512
+ * (the VAE's attention) run its tiled matrix-core kernels. */
 const char* sdxl_attn_kernel_name(int32_t resolved_backend);
 
 const char* sdxl_status_string(sdxl_status status);

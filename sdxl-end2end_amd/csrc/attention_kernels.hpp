@@ -74,6 +74,11 @@ struct OnlineAttentionParams {
 // dtype: 0 f16, 1 bf16, 2 f32 (sdxl_dtype values).
 hipError_t launch_online_attention(const OnlineAttentionParams& params, int dtype, hipStream_t stream);
 
+// Tiled attention on the 16-bit matrix cores with operands and probabilities as
+// 16-bit planes (fp32 accuracy): every dtype, head_dim <= 160, key masks, causal.
+bool tiled_attention_eligible(const OnlineAttentionParams& params, int dtype);
+hipError_t launch_tiled_attention(const OnlineAttentionParams& params, int dtype, int compute_units, hipStream_t stream);
+
 // FP32 head_dim 512 on the fp32 matrix cores (the VAE mid-block attention):
 // non-causal, unmasked, 16-byte aligned rows. Same parameters as the online kernel.
 bool attention_f32_d512_eligible(const OnlineAttentionParams& params, int dtype);

@@ -220,9 +220,12 @@ sdxl_status sdxl_attn_fwd(const sdxl_attn_desc* d, const void* q, const void* k,
         p.scale = scale;
         // FP32 at head_dim 512 (the VAE's attention) runs on the fp32 matrix
         // cores when the call allows (auto backend, no mask, non-causal,
-        // aligned rows); an explicit warp-online request keeps the per-row kernel.
+        // aligned rows), head_dim <= 160 on the tiled kernel; an explicit
+        // warp-online request keeps the per-row kernel.
         if (d->backend == SDXL_ATTN_AUTO && sdxl_hip::attention_f32_d512_eligible(p, d->dtype))
             err = sdxl_hip::launch_attention_f32_d512(p, compute_units(), s);
+        else if (d->backend == SDXL_ATTN_AUTO && sdxl_hip::tiled_attention_eligible(p, d->dtype))
+            err = sdxl_hip::launch_tiled_attention(p, d->dtype, compute_units(), s);
         else err = sdxl_hip::launch_online_attention(p, d->dtype, s);
     } else {
         sdxl_hip::FusedAttentionParams p{};

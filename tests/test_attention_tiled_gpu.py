@@ -1,0 +1,115 @@
+"""The tiled kernel of the online family (head_dim <= 160, every dtype) against 64-bit attention and
+the per-row kernel: edges of its key sub-tiles, query blocks and padded head dimensions, its three
+workgroup forms, masks, causal limits, unaligned rows, and values its 16-bit planes cannot carry."""
+import pytest
+
+import sdxl_hip as sh
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+DTYPES = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+# Half a unit of the output's last place, relative (none for FP32 beyond the absolute bound).
+OUT_ROUNDING = {"f32": 2.0 ** -24, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+# Scores: sums of D <= 160 products of N(0,1) values, |score| < 8 after scaling, each within
+# sqrt(160) * 2^-24 * 8 < 1e-5 of the exact one; probabilities move by that relative error and the
+# output by its share of max |v| < 5, less the averaging over keys.
+ABS = 2e-5
+
+
+def tensors(seed, B, H, Sq, Sk, D, dtype):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    make = lambda s: torch.randn(B, s, H * D, device=DEV, generator=g).to(DTYPES[dtype])
+    return make(Sq), make(Sk), make(Sk)
+
+
+def reference(q, k, v, H, causal=False, key_mask=None):
+    B, Sq, W = q.shape
+    Sk, D = k.shape[1], W // H
+    out = torch.zeros(B, Sq, W, dtype=torch.float64, device=DEV)
+    for b in range(B):
+        for h in range(H):
+            c = slice(h * D, (h + 1) * D)
+            s = q[b, :, c].double() @ k[b, :, c].double().t() / D ** 0.5
+            if key_mask is not None:
+                s.masked_fill_(key_mask[b][None] == 0, float("-inf"))
+            if causal:
+                s.masked_fill_(torch.ones(Sq, Sk, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+            out[b, :, c] = torch.nan_to_num(torch.softmax(s, -1)) @ v[b, :, c].double()
+    return out
+
+
+def check(got, ref, dtype):
+    err = (got.double() - ref).abs() - OUT_ROUNDING[dtype] * ref.abs()
+    assert err.max().item() <= ABS, err.max().item()
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("B,H,Sq,Sk,D", [
+    (1, 1, 1, 1, 8), (2, 3, 31, 33, 16), (1, 2, 65, 64, 32), (1, 2, 129, 65, 40),
+    (1, 3, 64, 127, 64), (2, 2, 63, 128, 72), (1, 2, 130, 129, 96), (1, 2, 33, 200, 128),
+    (1, 2, 70, 31, 136), (2, 1, 97, 300, 160),
+    (1, 3, 50, 77, 7), (1, 2, 66, 90, 33), (2, 2, 40, 70, 50), (1, 2, 35, 100, 159),  # rows not 16-byte aligned
+    (2, 40, 1000, 70, 40), (1, 20, 900, 260, 64)])  # one and two key groups on full grids
+def test_tiled_shapes(B, H, Sq, Sk, D, dtype):
+    if dtype != "f32" and D == 64:
+        D = 56  # 16-bit head_dim 64 runs elsewhere
+    q, k, v = tensors(B + Sq + D, B, H, Sq, Sk, D, dtype)
+    for causal in (False, True):
+        check(sh.attention(q, k, v, H, causal=causal), reference(q, k, v, H, causal), dtype)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("causal", [False, True])
+def test_tiled_key_mask(dtype, causal):
+    B, H, Sq, Sk, D = 3, 2, 150, 170, 80
+    q, k, v = tensors(5, B, H, Sq, Sk, D, dtype)
+    g = torch.Generator(device=DEV).manual_seed(6)
+    mask = (torch.rand(B, Sk, device=DEV, generator=g) < 0.6).int()
+    mask[0, :100] = 0  # whole sub-tiles hidden, and with causal whole rows
+    mask[1] = 0        # nothing visible: zeros
+    got = sh.attention(q, k, v, H, causal=causal, key_mask=mask)
+    check(got, reference(q, k, v, H, causal, mask), dtype)
+    assert (got[1] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_tiled_unaligned_and_strided_rows(dtype):
+    """head_dim 64 and 48 as slices of wider rows, aligned and off by one element."""
+    for D, offset in ((64 if dtype == "f32" else 48, 8), (48, 1), (64, 3)):
+        B, H, S = 2, 3, 75
+        wide = torch.randn(B, S, 3 * H * D + 17, device=DEV, generator=torch.Generator(device=DEV).manual_seed(D)).to(DTYPES[dtype])
+        q, k, v = (wide[..., offset + i * H * D: offset + (i + 1) * H * D] for i in range(3))
+        check(sh.attention(q, k, v, H), reference(q, k, v, H), dtype)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.3e38, 3.402e38])
+def test_tiled_values_planes_cannot_carry(dtype, where, value):
+    """Infinities, NaN and FP32 values above the largest bf16 give what the per-row kernel gives."""
+    B, H, Sq, Sk, D = 1, 2, 70, 100, 72
+    q, k, v = tensors(9, B, H, Sq, Sk, D, dtype)
+    {"q": q, "k": k, "v": v}[where][0, 57, D + 3] = value
+    got = sh.attention(q, k, v, H).float()
+    ref = sh.attention(q, k, v, H, backend=sh.WARP_ONLINE).float()
+    torch.testing.assert_close(got, ref, rtol=2.0 ** -7 if dtype == "bf16" else 2e-3, atol=1e-3, equal_nan=True)
+
+
+def test_tiled_large_logits():
+    """Logits of a few hundred, rising along the keys: the running maximum moves in every sub-tile."""
+    B, H, S, D = 1, 2, 300, 64
+    q, k, v = tensors(11, B, H, S, S, D, "f32")
+    q = q * 16
+    k = k * torch.linspace(1, 6, S, device=DEV)[None, :, None]
+    # a score error of 2^-24 * 160 * |score| (< 600) moves a probability by up to 6e-3 at worst;
+    # sums of rounding errors are far smaller: sqrt(64) * 2^-24 * 600 * max |v|
+    err = (sh.attention(q, k, v, H).double() - reference(q, k, v, H)).abs().max().item()
+    assert err <= 8 * 2.0 ** -24 * 600 * 5, err
+
+
+@pytest.mark.parametrize("D", [160, 161])
+def test_tiled_limit_of_the_head_dimension(D):
+    q, k, v = tensors(13, 1, 2, 40, 50, D, "f32")
+    check(sh.attention(q, k, v, 2), reference(q, k, v, 2), "f32")
