@@ -1,423 +1,564 @@
-// FP32 attention at head dimension 512 on the fp32 matrix cores.
+// FP32 attention at head dimension 512.
 //
 // The SDXL VAE decoder's mid-block attention is single-head with the head
 // width equal to the 512 channels, in FP32 (reference src/cuda/vae.cpp:65-99,
 // dispatched to generic_online_attention_f32_kernel,
 // src/cuda/ops_kernels.cu:1355-1419: one block per query, keys one by one).
-// At a 128x128 latent that is 16384 tokens: 550 GFLOP per call, which the
-// per-row online kernels run at ~3 TFLOP/s. This kernel is a tiled online
-// softmax on v_mfma_f32_32x32x2_f32 with the same semantics (exact fp32
-// products, fp32 accumulation, softmax with a running maximum, output divided
-// by max(sum, 1e-20)); non-causal, unmasked calls with 16-byte aligned rows.
+// At a 128x128 latent that is 16384 tokens: 550 GFLOP per call. Same semantics
+// (softmax with a running maximum, output divided by max(sum, 1e-20));
+// non-causal, unmasked calls with 16-byte aligned rows.
 //
-// Work split: a workgroup = 8 waves = 64 queries of one (batch, head): wave
-// w = 4 qt + dq owns query tile qt (32 rows) and head-dimension quarter dq
-// (128 dims) of the output, O^T[d][q] in 4 MFMA tiles (64 VGPRs). Per block
-// of 32 keys:
-//   * the 32 x 512 fp32 K tile (64 KiB) moves HBM -> LDS by DMA, double
-//     buffered (128 KiB), chunks XOR-swizzled by row so that the 32 rows'
-//     16-byte reads at one column hit distinct banks;
-//   * each wave forms the partial scores S^T = K[:, dq] Q[:, dq]^T over its
-//     128 dims (64 MFMAs), the four partials of a query tile are summed in a
-//     fixed order through LDS (16 KiB per tile, 32 KiB), so every wave of the
-//     tile holds the same full scores;
-//   * online softmax per query (the C layout gives each lane one query with
-//     16 of the 32 keys; the other 16 sit in lane l ^ 32);
-//   * O^T[d][q] += V^T P^T for the wave's 128 dims (64 MFMAs): V rows come
-//     straight from global memory (lane l reads 4 consecutive dims of one key
-//     row: the 4 accumulator tiles hold dims 128 dq + 4 m + t, t = 0..3), and
-//     P^T from the score registers, MFMA j pairing the keys held in register
-//     j by the two lane halves (the reduction order over keys is free).
-// The reduction order over the head dimension in S is likewise permuted
-// (MFMA j of group g pairs dims 8g + j and 8g + 4 + j), so every lane loads
-// its K and Q operands as 16-byte chunks.
+// Arithmetic: operands are split exactly into three bf16 planes and a product
+// is six plane products on the bf16 matrix cores (attention_planes.hpp), 2.7x
+// the fp32 matrix cores' rate; all sums are fp32.
+//
+// Work split: a workgroup = 8 waves = 32 kQT queries of one (batch, head);
+// wave w owns dims 64 w .. +63 of the scores for all of the queries: its slice
+// of Q as planes in registers (kQT = 2: the third plane in LDS) and of K,
+// which, like its 32 kDT dims of V, comes straight from global memory in the
+// matrix operands' layout, so that each element is split by one wave only.
+// With kDT = 1 two workgroups share a query block, each with half of the
+// output's dims. Per block of 32 keys t:
+//   * the partial scores S^T over the wave's 64 dims, formed one block ahead,
+//     meet in LDS; each wave sums the eight partials of 4 kQT queries (lane
+//     groups of 16 / kQT lanes share a query, its maximum and sum are DPP
+//     reductions), forms their probabilities once, and leaves them in LDS as
+//     planes, with the factor by which the maximum's move scales O;
+//   * meanwhile the waves form the partial scores of block t + 1;
+//   * O^T[d][q] += V^T P^T for the wave's output dims.
+// Two barriers per block. Each stage of a block is the matrix instructions of
+// one operand (12 or 6) with the split of the next operand and the stage's
+// share of the other work issued between them: the waves of a SIMD run in
+// step, and with the splits in front of the matrix instructions neither unit
+// worked while the other did (3.33 against 2.73 ms at 16384 tokens).
+//
+// Bound: at 64 queries the bf16 matrix cores, busy 72 % of a block's ~8500
+// cycles at a power-limited ~1.7 GHz (1.29 PFLOP/s of plane products; the
+// vendor's bf16 GEMM reaches 1.16 on the same card); at 32 the split's vector
+// instructions and the exchange of the partials (MFMA 3072 of ~6800 cycles).
+// Measured against fp32 matrix instructions (v_mfma_f32_32x32x2, the same
+// outputs within 64-bit error 2.0e-6 here, 2.3e-6 there): 16384 tokens 5.02 ->
+// 2.56 ms (215 TFLOP/s), 8192 1.43 -> 0.89, 4096 0.403 -> 0.349 (two
+// workgroups per block; one: 0.400), 1024 105 -> 83 us. Tried and not kept:
+// the residuals x - h by v_dot2 (fewer instructions, but wait states: 2.92
+// ms), K loads of 64-byte row segments exchanged by v_permlane16_swap (4096
+// tokens 421 -> 435 us).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "attention_kernels.hpp"
+#include "attention_planes.hpp"
 
 namespace sdxl_hip {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) char lds_char;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef __attribute__((address_space(3))) float lds_float;
 
 constexpr int kDim = 512;
-constexpr int kKeys = 32;                        // keys per block
-constexpr int kRowBytes = kDim * 4;              // 2 KiB per K row
-constexpr int kTileBytes = kKeys * kRowBytes;    // 64 KiB per K tile
-constexpr int kPartFloats = 16 * 64;             // one wave's partial scores
+constexpr int kKeys = 32;   // keys per block
+constexpr int kWaves = 8;
+constexpr int kSlice = 64;  // dims per wave
 
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const lds_char*)p; }
-
-// One 1-KiB HBM -> LDS transfer: lane l copies 16 bytes from base + voff to
-// LDS byte lds + 16 l (base and lds wave-uniform, M0 holds the destination).
-// Inline assembly keeps the compiler from ordering it against LDS reads or
-// waiting on it; the kernel orders it explicitly (vmcnt(0) and a barrier
-// before a tile is read, the transfer into a buffer only after the barrier
-// that ends the buffer's previous reads).
-__device__ __forceinline__ void lds_dma16(const char* base, uint32_t voff, uint32_t lds) {
-    const uint64_t b = (uint64_t)(uintptr_t)base;
-    const uint64_t ub = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32) |
-                        (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
-    base = (const char*)(uintptr_t)ub;
-    lds = __builtin_amdgcn_readfirstlane(lds);
-    asm volatile(
-        "s_nop 4\n\t"
-        "global_load_lds_dwordx4 %0, %1"
-        :
-        : "v"(voff), "s"(base), "{m0}"(lds));
+template <int kCtrl>
+__device__ __forceinline__ float dpp(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), kCtrl, 0xF, 0xF, true));
+}
+// Maximum and sum over groups of 8 (kN = 8) or 16 consecutive lanes, in all of them.
+template <int kN>
+__device__ __forceinline__ float group_max(float x) {
+    x = fmaxf(x, dpp<0xB1>(x));   // quad_perm 1,0,3,2
+    x = fmaxf(x, dpp<0x4E>(x));   // quad_perm 2,3,0,1
+    x = fmaxf(x, dpp<0x141>(x));  // row_half_mirror
+    if constexpr (kN == 16) x = fmaxf(x, dpp<0x140>(x));  // row_mirror
+    return x;
+}
+template <int kN>
+__device__ __forceinline__ float group_sum(float x) {
+    x += dpp<0xB1>(x);
+    x += dpp<0x4E>(x);
+    x += dpp<0x141>(x);
+    if constexpr (kN == 16) x += dpp<0x140>(x);
+    return x;
 }
 
-__device__ __forceinline__ void wait_vmem_all() { __builtin_amdgcn_s_waitcnt(0x0070); }  // vmcnt(0)
+// 64 kN dims of one output row in plain fp32 by a wave, for the calls whose
+// values planes cannot carry: as the per-row kernel, a NaN score making the
+// row NaN. v and o point at the first of those dims.
+template <int kN>
+__device__ __attribute__((noinline)) void plain_row(const float* q, const float* k, const float* v, float* o, int64_t k_stride,
+                                                    int64_t v_stride, int k_seq, float scale) {
+    const int lane = threadIdx.x & 63;
+    float acc[kN];
+    for (int i = 0; i < kN; ++i) acc[i] = 0.0f;
+    float m = -__builtin_inff(), l = 0.0f;
+    bool nan = false;
+#pragma unroll 1
+    for (int k0 = 0; k0 < k_seq; k0 += 64) {
+        const float* key = k + (int64_t)min(k0 + lane, k_seq - 1) * k_stride;
+        float s = 0.0f;
+#pragma unroll 1
+        for (int d = 0; d < kDim; ++d) s += q[d] * key[d];
+        s *= scale;
+        if (k0 + lane >= k_seq) s = -__builtin_inff();
+        nan = nan || __builtin_amdgcn_ballot_w64(s != s) != 0;
+        float mx = s;
+        for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+        const float m_new = fmaxf(m, mx);
+        if (m_new == -__builtin_inff()) continue;
+        const float alpha = m == -__builtin_inff() ? 0.0f : expf(m - m_new);
+        const float pr = k0 + lane < k_seq ? expf(s - m_new) : 0.0f;
+        float sum = pr;
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        l = l * alpha + sum;
+        m = m_new;
+        for (int i = 0; i < kN; ++i) acc[i] *= alpha;
+        const int n = min(64, k_seq - k0);
+#pragma unroll 1
+        for (int j = 0; j < n; ++j) {
+            const float pj = __shfl(pr, j, 64);
+            for (int i = 0; i < kN; ++i) acc[i] += pj * v[(int64_t)(k0 + j) * v_stride + lane + 64 * i];
+        }
+    }
+    const float inv = nan ? __builtin_nanf("") : 1.0f / fmaxf(l, 1.0e-20f);
+    for (int i = 0; i < kN; ++i) o[lane + 64 * i] = acc[i] * inv;
+}
 
-__device__ __forceinline__ float xhalf_max(float x) { return fmaxf(x, __shfl_xor(x, 32, 64)); }
-__device__ __forceinline__ float xhalf_sum(float x) { return x + __shfl_xor(x, 32, 64); }
+template <int kN> struct PerLane;
+template <> struct PerLane<2> { typedef f32x2 type; };
+template <> struct PerLane<4> { typedef f32x4 type; };
 
-// Physical 16-byte chunk of logical chunk c (0..127) in K row r: the low four
-// bits are XORed with r & 15, so 16 rows read at one logical chunk land in 16
-// distinct 16-byte bank groups.
-__device__ __forceinline__ int kchunk(int c, int r) { return c ^ (r & 15); }
-
-template <int N> struct FloatVec;
-template <> struct FloatVec<2> { typedef float type __attribute__((ext_vector_type(2))); };
-template <> struct FloatVec<4> { typedef float type __attribute__((ext_vector_type(4))); };
-
-// kQTiles = 32-query tiles per workgroup, kSlices = slices of the head
-// dimension (512 / kSlices dims per wave): (2, 4) = 8 waves for calls with at
-// least as many 64-query blocks as CUs, else (1, 4) = 4 waves (measured at
-// 4096 tokens: 0.71 ms; (1, 8), two waves per SIMD on one query tile, 0.85).
-template <int kQTiles, int kSlices>
-__global__ __launch_bounds__(kQTiles * kSlices * 64, 1) void attention_f32_d512_kernel(OnlineAttentionParams p, int q_blocks) {
-    constexpr int kWaves = kQTiles * kSlices;
-    constexpr int kPerWave = 64 / kWaves;  // 1-KiB K transfers per wave and tile
-    constexpr int kSD = kDim / kSlices;    // dims per wave
-    constexpr int kTD = kSD / 32;          // accumulator tiles per wave (dims kSD dq + kTD m + t)
-    constexpr int kG = kSD / 8;            // 4-MFMA groups of the partial scores
-    typedef typename FloatVec<kTD>::type vtype;
-    static_assert(kWaves * kPartFloats * 4 + 2 * kTileBytes <= 160 * 1024, "LDS");
-    __shared__ __attribute__((aligned(16))) char kbuf[2][kTileBytes];
-    __shared__ __attribute__((aligned(16))) float part[kWaves][kPartFloats];
+template <int kQT, int kDT>
+__global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(OnlineAttentionParams p, int q_blocks) {
+    constexpr int kSteps = kSlice / 16;          // K steps of a partial score
+    constexpr int kParts = 2 / kDT;              // workgroups that share a query block's output
+    constexpr int kRegPlanes = kQT == 2 ? 2 : 3; // Q planes in registers
+    constexpr int kPer = 2 * kQT;                // scores per lane of the summed block
+    constexpr int kGroup = kKeys / kPer;         // lanes per query there
+    constexpr int kPartBytes = kWaves * kQT * 4 * 1024;
+    constexpr int kQlBytes = kQT == 2 ? kWaves * kQT * kSteps * 1024 : 0;
+    constexpr int kProbBytes = kQT * 2 * 3 * 1024;
+    __shared__ __attribute__((aligned(16))) char part[kPartBytes];  // [wave][tile][4][64] x 16 bytes
+    __shared__ __attribute__((aligned(16))) char qlow[kQlBytes + 16];
+    __shared__ __attribute__((aligned(16))) char prob[kProbBytes];  // [tile][16-key half][plane][64] x 16 bytes
+    __shared__ float scale_o[32 * kQT];
+    __shared__ float total[32 * kQT];
+    __shared__ int special;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int qt = wave / kSlices, dq = wave % kSlices;
     const int hf = lane >> 5, col = lane & 31;
-
-    const int bh = blockIdx.x / q_blocks;
-    const int q0 = (blockIdx.x % q_blocks) * (32 * kQTiles) + 32 * qt;
+    const int task = blockIdx.x / kParts, out_part = blockIdx.x % kParts;
+    const int bh = task / q_blocks;
+    const int q0 = (task % q_blocks) * (32 * kQT);
     const int h = bh % p.heads, b = bh / p.heads;
-    const float* qbase = (const float*)p.q + ((int64_t)b * p.q_seq * p.q_row_stride + (int64_t)h * kDim);
-    const char* kbase = (const char*)((const float*)p.k + ((int64_t)b * p.k_seq * p.k_row_stride + (int64_t)h * kDim));
-    const float* vbase = (const float*)p.v + ((int64_t)b * p.k_seq * p.v_row_stride + (int64_t)h * kDim);
-    float* obase = (float*)p.o + ((int64_t)b * p.q_seq * p.o_row_stride + (int64_t)h * kDim);
+    const float* qhead = (const float*)p.q + ((int64_t)b * p.q_seq * p.q_row_stride + (int64_t)h * kDim);
+    const float* khead = (const float*)p.k + ((int64_t)b * p.k_seq * p.k_row_stride + (int64_t)h * kDim);
+    const float* vhead = (const float*)p.v + ((int64_t)b * p.k_seq * p.v_row_stride + (int64_t)h * kDim);
+    float* ohead = (float*)p.o + ((int64_t)b * p.q_seq * p.o_row_stride + (int64_t)h * kDim);
+    const char* kslice = (const char*)(khead + kSlice * wave);
+    const int out_dim = (kDim / kParts) * out_part + 32 * kDT * wave;  // this wave's first output dim
+    const char* vslice = (const char*)(vhead + out_dim);
+    const uint32_t k_stride_b = (uint32_t)(p.k_row_stride * 4), v_stride_b = (uint32_t)(p.v_row_stride * 4);
     const int n_blocks = (p.k_seq + kKeys - 1) / kKeys;
-    const uint32_t k_stride_b = (uint32_t)(p.k_row_stride * 4);
 
-    // K tile of key block t into buffer buf: 64 transfers of 1 KiB, kPerWave
-    // per wave; transfer n fills physical chunks 64 (n & 1) .. +63 of row n >> 1.
-    // Rows past k_seq re-read the last key (their scores are masked).
-    auto issue_k = [&](int t, int buf) __attribute__((always_inline)) {
-        const char* src = kbase + (int64_t)t * kKeys * p.k_row_stride * 4;
-        const int last = p.k_seq - 1 - t * kKeys;
+    if (threadIdx.x == 0) special = 0;
+    __syncthreads();
+
+    // Buffer descriptor of the wave's slice of the rows of block t; rows past
+    // k_seq read zeros (K: their scores are hidden; V: zero probabilities).
+    auto block_rows = [&](const char* slice, uint32_t stride_b, int t, int dims) __attribute__((always_inline)) {
+        const int rows = min(kKeys, p.k_seq - t * kKeys);
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(slice + (int64_t)t * kKeys * stride_b), 0,
+                                                 (int)((uint32_t)(rows - 1) * stride_b + 4u * dims), 0x00027000);
+    };
+    // K of block t, K steps 2 half and 2 half + 1: lane holds key col, dims
+    // 16 ks + 8 hf .. +7 of the slice.
+    f32x4 kraw[kSteps][2];
+    const uint32_t k_off = (uint32_t)col * k_stride_b + 32u * hf;
+    auto load_k = [&](int t, int half) __attribute__((always_inline)) {
+        const auto rows = block_rows(kslice, k_stride_b, t, kSlice);
 #pragma unroll
-        for (int j = 0; j < kPerWave; ++j) {
-            const int n = wave * kPerWave + j;
-            const int row = n >> 1;
-            const int c = kchunk(64 * (n & 1) + lane, row);
-            const uint32_t off = (uint32_t)min(row, last) * k_stride_b + (uint32_t)(c << 4);
-            lds_dma16(src, off, lds_addr(&kbuf[buf][0] + 1024 * n));
+        for (int ks = 2 * half; ks < 2 * half + 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                kraw[ks][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, k_off, 64 * ks + 16 * i, 0));
+    };
+    // V of 16-key half ss of block t: lane holds keys 16 ss + 8 hf + e, dims
+    // kDT col .. + kDT - 1 of the slice.
+    float vraw[2][8][kDT];
+    const uint32_t v_off = 8u * hf * v_stride_b + 4u * kDT * col;
+    auto load_v = [&](int t, int ss) __attribute__((always_inline)) {
+        const auto rows = block_rows(vslice, v_stride_b, t, 32 * kDT);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if constexpr (kDT == 2) {
+                const f32x2 x = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rows, v_off, (16 * ss + e) * v_stride_b, 0));
+                vraw[ss][e][0] = x[0];
+                vraw[ss][e][1] = x[1];
+            } else {
+                vraw[ss][e][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, v_off, (16 * ss + e) * v_stride_b, 0));
+            }
         }
     };
-    issue_k(0, 0);
+    load_k(0, 0);
+    load_k(0, 1);
 
-    // Q^T operand: lane holds query q0 + col, dims kSD dq + 8g + 4hf .. +3 in
-    // qop[g] (MFMA j of group g takes element j).
-    f32x4 qop[kG];
-    {
-        const float* qrow = qbase + (int64_t)min(q0 + col, p.q_seq - 1) * p.q_row_stride + kSD * dq + 4 * hf;
+    // Q planes: lane holds query q0 + 32 qt + col, dims 16 ks + 8 hf .. +7.
+    i16x8 qop[kQT][kSteps][kRegPlanes];
+    char* const qlow_mine = qlow + (kQT == 2 ? wave * kQT * kSteps * 1024 : 0) + lane * 16;
 #pragma unroll
-        for (int g = 0; g < kG; ++g) qop[g] = *(const f32x4*)(qrow + 8 * g);
+    for (int qt = 0; qt < kQT; ++qt) {
+        const float* row = qhead + (int64_t)min(q0 + 32 * qt + col, p.q_seq - 1) * p.q_row_stride + kSlice * wave + 8 * hf;
+#pragma unroll
+        for (int ks = 0; ks < kSteps; ++ks) {
+            u32x4 pl[3];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f32x2 x = *(const f32x2*)(row + 16 * ks + 2 * i);
+                uint32_t w[3];
+                split2<3, false>(x[0], x[1], w);
+#pragma unroll
+                for (int j = 0; j < 3; ++j) pl[j][i] = w[j];
+            }
+#pragma unroll
+            for (int j = 0; j < kRegPlanes; ++j) qop[qt][ks][j] = __builtin_bit_cast(i16x8, pl[j]);
+            if constexpr (kQT == 2) *(lds_u32x4*)(qlow_mine + (qt * kSteps + ks) * 1024) = pl[2];
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 
+    f32x16 o[kQT][kDT];  // [tile][dt]: dims kDT m + dt of the slice, m the tile row
+#pragma unroll
+    for (int qt = 0; qt < kQT; ++qt)
+#pragma unroll
+        for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[qt][dt][i] = 0.0f;
+
+    // Planes of the next matrix operand, formed while the matrix cores work on
+    // the current one (two sets in turn).
+    struct Operand { i16x8 pl[3]; };
+    auto split8 = [&](const float (&x)[8]) __attribute__((always_inline)) {
+        u32x4 pl[3];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t w[3];
+            split2<3, false>(x[2 * i], x[2 * i + 1], w);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) pl[j][i] = w[j];
+        }
+        return Operand{{__builtin_bit_cast(i16x8, pl[0]), __builtin_bit_cast(i16x8, pl[1]), __builtin_bit_cast(i16x8, pl[2])}};
+    };
+    auto split_k = [&](int ks) __attribute__((always_inline)) {
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = kraw[ks][i >> 2][i & 3];
+        return split8(x);
+    };
+    auto split_v = [&](int ss, int dt) __attribute__((always_inline)) {
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = vraw[ss][i][dt];
+        return split8(x);
+    };
+    // partial scores, K step ks
+    f32x16 s[kQT];
+    i16x8 qlo[kQT];  // third plane of Q, read from LDS a stage ahead
+    auto read_qlow = [&](int ks) __attribute__((always_inline)) {
+        if constexpr (kQT == 2)
+#pragma unroll
+            for (int qt = 0; qt < kQT; ++qt) qlo[qt] = __builtin_bit_cast(i16x8, *(const lds_u32x4*)(qlow_mine + (qt * kSteps + ks) * 1024));
+    };
+    auto scores_step = [&](int ks, const Operand& k, const i16x8 (&low)[kQT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int qt = 0; qt < kQT; ++qt) {
+            i16x8 ql;
+            if constexpr (kQT == 2) ql = low[qt];
+            else ql = qop[qt][ks][2];
+            s[qt] = mfma32<false>(k.pl[2], qop[qt][ks][0], s[qt]);
+            s[qt] = mfma32<false>(k.pl[1], qop[qt][ks][1], s[qt]);
+            s[qt] = mfma32<false>(k.pl[1], qop[qt][ks][0], s[qt]);
+            s[qt] = mfma32<false>(k.pl[0], ql, s[qt]);
+            s[qt] = mfma32<false>(k.pl[0], qop[qt][ks][1], s[qt]);
+            s[qt] = mfma32<false>(k.pl[0], qop[qt][ks][0], s[qt]);
+        }
+    };
+    // O^T of dims dt += V^T P^T over a 16-key half
+    struct Probs { i16x8 pl[kQT][3]; };
+    auto read_probs = [&](int ss) __attribute__((always_inline)) {
+        Probs r;
+#pragma unroll
+        for (int qt = 0; qt < kQT; ++qt)
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl)
+                r.pl[qt][pl] = __builtin_bit_cast(i16x8, *(const lds_u32x4*)(prob + ((qt * 2 + ss) * 3 + pl) * 1024 + lane * 16));
+        return r;
+    };
+    auto output_step = [&](int dt, const Operand& v, const Probs& probs) __attribute__((always_inline)) {
+#pragma unroll
+        for (int qt = 0; qt < kQT; ++qt) {
+            const i16x8 (&pop)[3] = probs.pl[qt];
+            o[qt][dt] = mfma32<false>(v.pl[2], pop[0], o[qt][dt]);
+            o[qt][dt] = mfma32<false>(v.pl[1], pop[1], o[qt][dt]);
+            o[qt][dt] = mfma32<false>(v.pl[0], pop[2], o[qt][dt]);
+            o[qt][dt] = mfma32<false>(v.pl[1], pop[0], o[qt][dt]);
+            o[qt][dt] = mfma32<false>(v.pl[0], pop[1], o[qt][dt]);
+            o[qt][dt] = mfma32<false>(v.pl[0], pop[0], o[qt][dt]);
+        }
+    };
+    // Ends a stage: its matrix instructions spread over its other work, kValu
+    // vector instructions after each.
+    auto stage_end = [&]<int kValu>() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 6 * kQT; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);  // VALU
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto clear_scores = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int qt = 0; qt < kQT; ++qt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[qt][i] = 0.0f;
+    };
+    // Partials: element 4u + r is key 8u + 4hf + r of query col; 16-byte unit
+    // (hf, col) of [tile][u] sits at column col ^ 2 (2u + hf), so that the
+    // summing lanes (8 units of one column each) reach distinct banks.
+    auto write_partials = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int qt = 0; qt < kQT; ++qt)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                char* dst = part + ((wave * kQT + qt) * 4 + u) * 1024 + (32 * hf + (col ^ (2 * (2 * u + hf)))) * 16;
+                *(lds_f32x4*)dst = f32x4{s[qt][4 * u], s[qt][4 * u + 1], s[qt][4 * u + 2], s[qt][4 * u + 3]};
+            }
+    };
+
+    // This lane's share of the summed scores: query sq of tile st, keys
+    // 8 su + 4 sh + sr .. + kPer - 1.
+    const int j = lane % kGroup;
+    const int st = kQT == 2 ? wave >> 2 : 0;
+    const int sq = (64 / kGroup) * (kQT == 2 ? wave & 3 : wave) + lane / kGroup;
+    const int su = kQT == 2 ? j >> 1 : j >> 2, sh = kQT == 2 ? j & 1 : (j >> 1) & 1, sr = kQT == 2 ? 0 : 2 * (j & 1);
+    const char* const part_mine = part + (st * 4 + su) * 1024 + (32 * sh + (sq ^ (2 * (2 * su + sh)))) * 16 + 4 * sr;
+    // B operand of P.V: 16-key half ss, lane (hf', query): keys 16 ss + 8 hf' + e
+    char* const prob_mine = prob + (st * 2 + (su >> 1)) * 3 * 1024 + (32 * (su & 1) + sq) * 16 + 8 * sh + 2 * sr;
     const float c = p.scale * 1.4426950408889634f;  // scores to log2 units
-    f32x16 o[kTD];
-#pragma unroll
-    for (int t = 0; t < kTD; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[t][i] = 0.0f;
-    float m_run = -__builtin_inff();  // running maximum (log2 units) of this lane's query
-    float l_run = 0.0f;               // this lane's half of the running sum
-    const float* vcol = vbase + kSD * dq + kTD * col;
-    // K operand address: lane reads row col, logical chunk (kSD / 4) dq + 2g + hf.
-    const int krow_off = col * kRowBytes;
+    float m_run = -__builtin_inff(), l_run = 0.0f;  // of query sq; this lane's part of the sum
 
-    for (int t = 0; t < n_blocks; ++t) {
-        const int buf = t & 1;
-        wait_vmem_all();  // this wave's part of K(t) landed
-        __syncthreads();  // all of K(t); every wave is done with K(t - 1) and the partial scores
-        if (t + 1 < n_blocks) issue_k(t + 1, buf ^ 1);
-
-        // V rows of this block for PV: register j holds key 8(j >> 2) + 4hf +
-        // (j & 3), dims kSD dq + kTD col .. +kTD-1. The first half is loaded now (in
-        // flight during S), the second after S (in flight during the score
-        // reduction, the softmax and the first half of PV).
-        vtype vop[16];
-        auto load_v = [&](int j0) __attribute__((always_inline)) {
-            const int key0 = t * kKeys;
+    float sc[kPer];
+    typedef typename PerLane<kPer>::type part_t;
+    part_t parts[kWaves / 2];
+    auto read_partials = [&](int half) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = j0; j < j0 + 8; ++j) {
-                const int key = min(key0 + 8 * (j >> 2) + 4 * hf + (j & 3), p.k_seq - 1);
-                vop[j] = *(const vtype*)(vcol + (int64_t)key * p.v_row_stride);
-            }
-        };
-        load_v(0);
-
-        // partial S^T over this wave's kSD dims
-        // two accumulator chains (even and odd groups), summed after: at 16384
-        // tokens 5.12 -> 5.00 ms against one chain (the same interleave in the
-        // 16-query kernel measured slower, 399 -> 416 us at 4096 tokens)
-        f32x16 s, s_odd;
+        for (int w = 0; w < kWaves / 2; ++w)
+            parts[w] = *(const __attribute__((address_space(3))) part_t*)(part_mine + (half * (kWaves / 2) + w) * (kQT * 4 * 1024));
+    };
+    auto sum_partials = [&](int half) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = s_odd[i] = 0.0f;
-        const char* kt = &kbuf[buf][0] + krow_off;
-#pragma unroll
-        for (int g = 0; g < kG; g += 2) {
-            const f32x4 kop0 = *(const lds_f32x4*)(kt + (kchunk((kSD / 4) * dq + 2 * g + hf, col) << 4));
-            const f32x4 kop1 = *(const lds_f32x4*)(kt + (kchunk((kSD / 4) * dq + 2 * (g + 1) + hf, col) << 4));
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kop0[j], qop[g][j], s, 0, 0, 0);
-                s_odd = __builtin_amdgcn_mfma_f32_32x32x2f32(kop1[j], qop[g + 1][j], s_odd, 0, 0, 0);
-            }
+        for (int i = 0; i < kPer; ++i) {
+            const float x = (parts[0][i] + parts[1][i]) + (parts[2][i] + parts[3][i]);
+            sc[i] = half == 0 ? x : sc[i] + x;
         }
-        s += s_odd;
-        load_v(8);
-        float* mine = &part[wave][0];
+    };
+    auto softmax = [&](int t) __attribute__((always_inline)) {
+        const int lim = p.k_seq - t * kKeys - (8 * su + 4 * sh + sr);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mine[i * 64 + lane] = s[i];
-        __syncthreads();
-        // full scores: the tile's partials in dq order (the same sum in every wave of the tile)
+        for (int i = 0; i < kPer; ++i) sc[i] = i < lim ? sc[i] : -__builtin_inff();
+        float mx = sc[0];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float acc = part[kSlices * qt][i * 64 + lane];
-#pragma unroll
-            for (int w = 1; w < kSlices; ++w) acc += part[kSlices * qt + w][i * 64 + lane];
-            s[i] = acc;
-        }
-
-        // keys past k_seq: element i is key t*32 + 8(i >> 2) + 4hf + (i & 3)
-        const int lim = p.k_seq - t * kKeys - 4 * hf;
-        if (lim < 32) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] = 8 * (i >> 2) + (i & 3) < lim ? s[i] : -__builtin_inff();
-        }
-        float mx = -__builtin_inff();
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx = xhalf_max(mx) * c;
+        for (int i = 1; i < kPer; ++i) mx = fmaxf(mx, sc[i]);
+        mx = group_max<kGroup>(mx) * c;
         const float m_new = fmaxf(m_run, mx);  // finite: every block holds a visible key
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 on the first block
         m_run = m_new;
-        float pr[16];
-        float sum = 0.0f;
+        float pr[kPer], sum = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            pr[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c, -m_new));
-            sum += pr[i];
-        }
-        l_run = l_run * alpha + sum;
-#pragma unroll
-        for (int tt = 0; tt < kTD; ++tt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o[tt][i] *= alpha;
-
-        // O^T[d][q] += V^T P^T: tile tt holds dims kSD dq + kTD m + tt
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-#pragma unroll
-            for (int tt = 0; tt < kTD; ++tt) o[tt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vop[j][tt], pr[j], o[tt], 0, 0, 0);
-    }
-
-    // ---- normalise and store: lane holds rows m = 8(i >> 2) + 4hf + (i & 3)
-    // of each tile for query q0 + col, i.e. dims kSD dq + kTD m .. +kTD-1.
-    const float inv = 1.0f / fmaxf(xhalf_sum(l_run), 1.0e-20f);
-    if (q0 + col < p.q_seq) {
-        float* orow = obase + (int64_t)(q0 + col) * p.o_row_stride + kSD * dq;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int m = 8 * (i >> 2) + 4 * hf + (i & 3);
-            vtype w;
-#pragma unroll
-            for (int tt = 0; tt < kTD; ++tt) w[tt] = o[tt][i] * inv;
-            *(vtype*)(orow + kTD * m) = w;
-        }
-    }
-}
-
-// Variant for calls with fewer 32-query tiles than CUs (the VAE at a 64x64
-// latent, 4096 tokens: 128 tiles): 16-query workgroups on
-// v_mfma_f32_16x16x4_f32, 4 waves = 4 slices of 128 dims, so twice as many
-// workgroups fill the CUs. Same algorithm and order of operations as above
-// per key block; the 16x16 C layout gives lane l query l & 15 and keys
-// 4 (l >> 4) .. +3 of each 16-key half, so the row maximum and sum take two
-// lane exchanges (l ^ 16, l ^ 32). Index maps (free reduction orders):
-//   S: MFMA j of group g pairs dim 16 g + 4 (l >> 4) + j of the slice (K and
-//      Q operands are 16-byte chunks);
-//   PV: score register r (key 16 (r >> 2) + 4 (l >> 4) + (r & 3)) is the B
-//      operand of MFMA r; accumulator tile tt row m holds dim 8 m + tt of the
-//      slice, so lane l loads dims 8 (l & 15) .. +7 of its key row (32 bytes)
-//      and stores 8 consecutive dims per register.
-__global__ __launch_bounds__(256, 1) void attention_f32_d512_q16_kernel(OnlineAttentionParams p, int q_blocks) {
-    constexpr int kWaves = 4;
-    constexpr int kPerWave = 64 / kWaves;
-    constexpr int kSD = kDim / kWaves;  // 128 dims per wave
-    static_assert(kWaves * 8 * 64 * 4 + 2 * kTileBytes <= 160 * 1024, "LDS");
-    __shared__ __attribute__((aligned(16))) char kbuf[2][kTileBytes];
-    __shared__ __attribute__((aligned(16))) float part[kWaves][8 * 64];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int dq = wave;
-    const int qc = lane & 15, kq = lane >> 4;
-
-    const int bh = blockIdx.x / q_blocks;
-    const int q0 = (blockIdx.x % q_blocks) * 16;
-    const int h = bh % p.heads, b = bh / p.heads;
-    const float* qbase = (const float*)p.q + ((int64_t)b * p.q_seq * p.q_row_stride + (int64_t)h * kDim);
-    const char* kbase = (const char*)((const float*)p.k + ((int64_t)b * p.k_seq * p.k_row_stride + (int64_t)h * kDim));
-    const float* vbase = (const float*)p.v + ((int64_t)b * p.k_seq * p.v_row_stride + (int64_t)h * kDim);
-    float* obase = (float*)p.o + ((int64_t)b * p.q_seq * p.o_row_stride + (int64_t)h * kDim);
-    const int n_blocks = (p.k_seq + kKeys - 1) / kKeys;
-    const uint32_t k_stride_b = (uint32_t)(p.k_row_stride * 4);
-
-    // K tile of key block t into buffer buf (as in the 32-query kernel).
-    auto issue_k = [&](int t, int buf) __attribute__((always_inline)) {
-        const char* src = kbase + (int64_t)t * kKeys * p.k_row_stride * 4;
-        const int last = p.k_seq - 1 - t * kKeys;
-#pragma unroll
-        for (int j = 0; j < kPerWave; ++j) {
-            const int n = wave * kPerWave + j;
-            const int row = n >> 1;
-            const int c = kchunk(64 * (n & 1) + lane, row);
-            const uint32_t off = (uint32_t)min(row, last) * k_stride_b + (uint32_t)(c << 4);
-            lds_dma16(src, off, lds_addr(&kbuf[buf][0] + 1024 * n));
-        }
-    };
-    issue_k(0, 0);
-
-    // Q operand: query q0 + qc, dims kSD dq + 16 g + 4 kq .. +3 in qop[g].
-    f32x4 qop[8];
-    {
-        const float* qrow = qbase + (int64_t)min(q0 + qc, p.q_seq - 1) * p.q_row_stride + kSD * dq + 4 * kq;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) qop[g] = *(const f32x4*)(qrow + 16 * g);
-    }
-
-    const float c = p.scale * 1.4426950408889634f;  // scores to log2 units
-    f32x4 o[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_run = -__builtin_inff();
-    float l_run = 0.0f;  // this lane's quarter of the running sum
-    const float* vcol = vbase + kSD * dq + 8 * qc;
-
-    for (int t = 0; t < n_blocks; ++t) {
-        const int buf = t & 1;
-        wait_vmem_all();
-        __syncthreads();
-        if (t + 1 < n_blocks) issue_k(t + 1, buf ^ 1);
-
-        // V operands: register r holds key t*32 + 16 (r >> 2) + 4 kq + (r & 3),
-        // dims kSD dq + 8 qc .. +7 (two 16-byte halves).
-        f32x4 vop[8][2];
-        auto load_v = [&](int r0) __attribute__((always_inline)) {
-#pragma unroll
-            for (int r = r0; r < r0 + 4; ++r) {
-                const int key = min(t * kKeys + 16 * (r >> 2) + 4 * kq + (r & 3), p.k_seq - 1);
-                const float* src = vcol + (int64_t)key * p.v_row_stride;
-                vop[r][0] = *(const f32x4*)src;
-                vop[r][1] = *(const f32x4*)(src + 4);
-            }
-        };
-        load_v(0);
-
-        f32x4 s[2];
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            s[kt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            const int row = 16 * kt + qc;
-            const char* krow = &kbuf[buf][0] + row * kRowBytes;
-#pragma unroll
-            for (int g = 0; g < 8; ++g) {
-                const f32x4 kop = *(const lds_f32x4*)(krow + (kchunk((kSD / 4) * dq + 4 * g + kq, row) << 4));
-#pragma unroll
-                for (int j = 0; j < 4; ++j) s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kop[j], qop[g][j], s[kt], 0, 0, 0);
-            }
-        }
-        load_v(4);
-        float* mine = &part[wave][0];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) mine[i * 64 + lane] = s[i >> 2][i & 3];
-        __syncthreads();
-        // full scores: the partials summed in slice order
-        float sc[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float acc = part[0][i * 64 + lane];
-#pragma unroll
-            for (int w = 1; w < kWaves; ++w) acc += part[w][i * 64 + lane];
-            sc[i] = acc;
-        }
-
-        // keys past k_seq: score i is key t*32 + 16 (i >> 2) + 4 kq + (i & 3)
-        const int lim = p.k_seq - t * kKeys - 4 * kq;
-        if (lim < 32) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) sc[i] = 16 * (i >> 2) + (i & 3) < lim ? sc[i] : -__builtin_inff();
-        }
-        float mx = -__builtin_inff();
-#pragma unroll
-        for (int i = 0; i < 8; ++i) mx = fmaxf(mx, sc[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c;
-        const float m_new = fmaxf(m_run, mx);  // finite: every block holds a visible key
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        m_run = m_new;
-        float pr[8];
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < kPer; ++i) {
             pr[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c, -m_new));
             sum += pr[i];
         }
         l_run = l_run * alpha + sum;
+        uint32_t w[kPer / 2][3];
 #pragma unroll
-        for (int tt = 0; tt < 8; ++tt) o[tt] *= alpha;
-
+        for (int i = 0; i < kPer / 2; ++i) split2<3, false>(pr[2 * i], pr[2 * i + 1], w[i]);
 #pragma unroll
-        for (int r = 0; r < 8; ++r)
-#pragma unroll
-            for (int tt = 0; tt < 8; ++tt)
-                o[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vop[r][tt >> 2][tt & 3], pr[r], o[tt], 0, 0, 0);
-    }
-
-    // ---- normalise and store: register i of tile tt is dim kSD dq + 8 (4 kq + i) + tt.
-    float l = l_run + __shfl_xor(l_run, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    const float inv = 1.0f / fmaxf(l, 1.0e-20f);
-    if (q0 + qc < p.q_seq) {
-        float* orow = obase + (int64_t)(q0 + qc) * p.o_row_stride + kSD * dq + 32 * kq;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const f32x4 lo = {o[0][i] * inv, o[1][i] * inv, o[2][i] * inv, o[3][i] * inv};
-            const f32x4 hi = {o[4][i] * inv, o[5][i] * inv, o[6][i] * inv, o[7][i] * inv};
-            *(f32x4*)(orow + 8 * i) = lo;
-            *(f32x4*)(orow + 8 * i + 4) = hi;
+        for (int pl = 0; pl < 3; ++pl) {
+            if constexpr (kQT == 2) *(lds_u32x2*)(prob_mine + pl * 1024) = u32x2{w[0][pl], w[1][pl]};
+            else *(lds_u32*)(prob_mine + pl * 1024) = w[0][pl];
         }
+        if (j == 0) scale_o[32 * st + sq] = alpha;
+    };
+
+    clear_scores();
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) {
+        read_qlow(ks);
+        scores_step(ks, split_k(ks), qlo);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    write_partials();
+    read_qlow(0);
+    Operand even = {}, odd = {};
+    if constexpr (kQT == 1) {
+        load_v(0, 0);
+        load_v(0, 1);
+    }
+    if (n_blocks > 1) {
+        load_k(1, 0);
+        load_k(1, 1);
+        even = split_k(0);
+    }
+    auto rescale = [&]() __attribute__((always_inline)) {
+        float alpha[kQT];
+        bool move = false;
+#pragma unroll
+        for (int qt = 0; qt < kQT; ++qt) {
+            alpha[qt] = scale_o[32 * qt + col];
+            move = move || alpha[qt] != 1.0f;
+        }
+        if (__builtin_amdgcn_ballot_w64(move) != 0) {
+#pragma unroll
+            for (int qt = 0; qt < kQT; ++qt)
+#pragma unroll
+                for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) o[qt][dt][i] *= alpha[qt];
+        }
+    };
+
+    // Block t: scores of t + 1, output of t (the last block has no next one).
+    constexpr int kFill = 8 / kQT;  // vector instructions per matrix instruction
+    auto scores_stage = [&]<int kStep>(const Operand& now, auto&& other) __attribute__((always_inline)) {
+        i16x8 low[kQT];
+#pragma unroll
+        for (int qt = 0; qt < kQT; ++qt) low[qt] = qlo[qt];
+        if constexpr (kStep + 1 < kSteps) read_qlow(kStep + 1);
+        other();
+        scores_step(kStep, now, low);
+        stage_end.template operator()<kStep == 2 ? 2 * kFill : kFill>();
+    };
+    for (int t = 0; t + 1 < n_blocks; ++t) {
+        // Loads: kQT = 1 a block ahead; kQT = 2, whose registers are full, two
+        // or three stages ahead, into what the last operands left. K of the
+        // block after next past the end: of the last block, unused.
+        const int t2 = min(t + 2, n_blocks - 1);
+        __syncthreads();  // partials of t there; probabilities of t - 1 used
+        clear_scores();
+        read_partials(0);
+        scores_stage.template operator()<0>(even, [&]() __attribute__((always_inline)) { odd = split_k(1); });
+        if constexpr (kQT == 2) load_v(t, 0);
+        else load_k(t2, 0);
+        sum_partials(0);
+        read_partials(1);
+        scores_stage.template operator()<1>(odd, [&]() __attribute__((always_inline)) { even = split_k(2); });
+        sum_partials(1);
+        scores_stage.template operator()<2>(even, [&]() __attribute__((always_inline)) {
+            odd = split_k(3);
+            softmax(t);
+        });
+        if constexpr (kQT == 2) load_v(t, 1);
+        else load_k(t2, 1);
+        scores_stage.template operator()<3>(odd, [&]() __attribute__((always_inline)) { even = split_v(0, 0); });
+        __syncthreads();  // probabilities of t there; partials of t used
+        Probs first = read_probs(0);
+        rescale();
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kQT == 2) load_k(t2, 0);
+        odd = split_v(kDT == 2 ? 0 : 1, kDT - 1);
+        output_step(0, even, first);
+        write_partials();
+        stage_end.template operator()<kFill>();
+        if constexpr (kQT == 1) load_v(t + 1, 0);
+        Probs second = read_probs(1);
+        if constexpr (kDT == 2) {
+            even = split_v(1, 0);
+            output_step(1, odd, first);
+            stage_end.template operator()<kFill>();
+            if constexpr (kQT == 2) load_k(t2, 1);
+            odd = split_v(1, 1);
+            output_step(0, even, second);
+            stage_end.template operator()<kFill>();
+        }
+        if constexpr (kQT == 1) load_v(t + 1, 1);
+        read_qlow(0);
+        even = split_k(0);
+        output_step(kDT - 1, odd, second);
+        stage_end.template operator()<kFill>();
+    }
+    __syncthreads();
+    if constexpr (kQT == 2) {
+        load_v(n_blocks - 1, 0);
+        load_v(n_blocks - 1, 1);
+    }
+    read_partials(0);
+    sum_partials(0);
+    read_partials(1);
+    sum_partials(1);
+    softmax(n_blocks - 1);
+    __syncthreads();
+    rescale();
+#pragma unroll
+    for (int ss = 0; ss < 2; ++ss)
+#pragma unroll
+        for (int dt = 0; dt < kDT; ++dt) {
+            output_step(dt, split_v(ss, dt), read_probs(ss));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+
+    l_run = group_sum<kGroup>(l_run);
+    if (j == 0) total[32 * st + sq] = l_run;
+    __syncthreads();
+    // Planes turn an infinity, a NaN or an FP32 value above the largest bf16
+    // into a NaN, which reaches every score or output that it meets: such
+    // workgroups (and those whose results overflow) start over in plain fp32.
+    float bad = 0.0f;
+#pragma unroll
+    for (int qt = 0; qt < kQT; ++qt) {
+        const float inv = 1.0f / fmaxf(total[32 * qt + col], 1.0e-20f);
+#pragma unroll
+        for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                o[qt][dt][i] *= inv;
+                bad = __builtin_fmaf(o[qt][dt][i], 0.0f, bad);
+            }
+    }
+    if (bad != bad) atomicOr(&special, 1);
+    __syncthreads();
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(special) != 0, 0)) {
+#pragma unroll 1
+        for (int r = wave; r < 32 * kQT; r += kWaves)
+            if (q0 + r < p.q_seq) {
+                const int first = (kDim / kParts) * out_part;
+                plain_row<kDim / kParts / 64>(qhead + (int64_t)(q0 + r) * p.q_row_stride, khead, vhead + first,
+                                              ohead + (int64_t)(q0 + r) * p.o_row_stride + first, p.k_row_stride, p.v_row_stride,
+                                              p.k_seq, p.scale);
+            }
+        return;
+    }
+    // lane holds tile rows m = 8u + 4hf + r of query col: dims kDT m + dt
+#pragma unroll
+    for (int qt = 0; qt < kQT; ++qt) {
+        const int query = q0 + 32 * qt + col;
+        if (query >= p.q_seq) continue;
+        float* row = ohead + (int64_t)query * p.o_row_stride + out_dim + 4 * kDT * hf;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int n = 0; n < 4 * kDT; n += 4) {
+                f32x4 w;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = o[qt][(n + i) % kDT][4 * u + (n + i) / kDT];
+                *(f32x4*)(row + 8 * kDT * u + n) = w;
+            }
     }
 }
 
@@ -428,27 +569,25 @@ bool attention_f32_d512_eligible(const OnlineAttentionParams& p, int dtype) {
     return dtype == 2 && p.head_dim == kDim && !p.causal && p.key_mask == nullptr && p.k_seq > 0 &&
            p.q_row_stride % 4 == 0 && p.k_row_stride % 4 == 0 && p.v_row_stride % 4 == 0 && p.o_row_stride % 4 == 0 &&
            a16(p.q) && a16(p.k) && a16(p.v) && a16(p.o) &&
-           (int64_t)kKeys * p.k_row_stride * 4 < (int64_t{1} << 31);
+           (int64_t)kKeys * p.k_row_stride * 4 < (int64_t{1} << 31) && (int64_t)kKeys * p.v_row_stride * 4 < (int64_t{1} << 31);
 }
 
 hipError_t launch_attention_f32_d512(const OnlineAttentionParams& p, int compute_units, hipStream_t stream) {
     if (p.batch == 0 || p.q_seq == 0) return hipSuccess;
-    // 64-query workgroups (waves: 2 query tiles x 4 dim slices) when they
-    // fill the CUs; else 32-query workgroups (1 x 4): twice the workgroups,
-    // each K tile staged for half as many queries; and when even those leave
-    // CUs idle, 16-query workgroups on the 16x16 matrix-core tiles.
+    // One workgroup per CU at a time. 64 queries per workgroup take 1.65x the
+    // time of 32 per key block (16384 tokens: 2.59 ms against 3.1 in two rounds
+    // of 32); with at most half the CUs' worth of 32-query blocks, two
+    // workgroups share a block's output dims (each forms all of its scores).
     const int64_t heads_total = (int64_t)p.heads * p.batch;
-    const int64_t blocks64 = (p.q_seq + 63) / 64 * heads_total;
-    const int cus = compute_units > 0 ? compute_units : 256;
-    const bool wide = blocks64 >= cus;
-    const bool q16 = !wide && (p.q_seq + 31) / 32 * heads_total < cus;
-    const int rows = wide ? 64 : q16 ? 16 : 32;
-    const int64_t q_blocks = (p.q_seq + rows - 1) / rows;
-    const int64_t grid = q_blocks * heads_total;
+    const int64_t cus = compute_units > 0 ? compute_units : 256;
+    const int64_t b64 = ((int64_t)p.q_seq + 63) / 64, b32 = ((int64_t)p.q_seq + 31) / 32;
+    const int64_t r64 = (b64 * heads_total + cus - 1) / cus, r32 = (b32 * heads_total + cus - 1) / cus;
+    const int64_t grid = (5 * r64 <= 3 * r32 ? b64 : 2 * b32 * heads_total <= cus ? 2 * b32 : b32) * heads_total;
     if (grid > INT32_MAX) return hipErrorInvalidValue;
-    if (q16) hipLaunchKernelGGL(attention_f32_d512_q16_kernel, dim3((unsigned)grid), dim3(256), 0, stream, p, (int)q_blocks);
-    else if (wide) hipLaunchKernelGGL((attention_f32_d512_kernel<2, 4>), dim3((unsigned)grid), dim3(512), 0, stream, p, (int)q_blocks);
-    else hipLaunchKernelGGL((attention_f32_d512_kernel<1, 4>), dim3((unsigned)grid), dim3(256), 0, stream, p, (int)q_blocks);
+    const dim3 g((unsigned)grid), block(kWaves * 64);
+    if (5 * r64 <= 3 * r32) hipLaunchKernelGGL((attention_f32_d512_kernel<2, 2>), g, block, 0, stream, p, (int)b64);
+    else if (2 * b32 * heads_total <= cus) hipLaunchKernelGGL((attention_f32_d512_kernel<1, 1>), g, block, 0, stream, p, (int)b32);
+    else hipLaunchKernelGGL((attention_f32_d512_kernel<1, 2>), g, block, 0, stream, p, (int)b32);
     return hipGetLastError();
 }
 

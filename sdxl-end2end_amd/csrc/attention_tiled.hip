@@ -40,19 +40,12 @@
 #include <stdint.h>
 
 #include "attention_kernels.hpp"
+#include "attention_planes.hpp"
 
 namespace sdxl_hip {
 namespace {
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef short i16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef __attribute__((address_space(3))) i16x8 lds_i16x8;
@@ -70,49 +63,6 @@ template <typename T> struct Planes;
 template <> struct Planes<float> { static constexpr int in = 3, prob = 3; static constexpr bool f16 = false; static constexpr float shift = 0.0f; };
 template <> struct Planes<__bf16> { static constexpr int in = 1, prob = 3; static constexpr bool f16 = false; static constexpr float shift = 0.0f; };
 template <> struct Planes<_Float16> { static constexpr int in = 1, prob = 2; static constexpr bool f16 = true; static constexpr float shift = 12.0f; };
-
-template <bool kF16>
-__device__ __forceinline__ f32x16 mfma32(i16x8 a, i16x8 b, f32x16 c) {
-    if constexpr (kF16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    const bf16x2 v = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(uint32_t, v);
-}
-__device__ __forceinline__ float lo_bf16(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
-__device__ __forceinline__ float hi_bf16(uint32_t v) { return __builtin_bit_cast(float, v & 0xFFFF0000u); }
-
-// Two values as kN planes: bf16 planes (exact for kN = 3) or two fp16 planes.
-template <int kN, bool kF16>
-__device__ __forceinline__ void split2(float a, float b, uint32_t (&out)[kN]) {
-    if constexpr (kF16) {
-        static_assert(kN == 2);
-        const f16x2 h = {(_Float16)a, (_Float16)b};
-        const f16x2 l = {(_Float16)(a - (float)h[0]), (_Float16)(b - (float)h[1])};
-        out[0] = __builtin_bit_cast(uint32_t, h);
-        out[1] = __builtin_bit_cast(uint32_t, l);
-    } else {
-#pragma unroll
-        for (int i = 0; i < kN; ++i) {
-            out[i] = pack_bf16(a, b);
-            if (i + 1 < kN) {
-                a -= lo_bf16(out[i]);
-                b -= hi_bf16(out[i]);
-            }
-        }
-    }
-}
-
-// NaN if the packed pair holds an infinity or a NaN, else x unchanged.
-template <bool kF16>
-__device__ __forceinline__ float probe(uint32_t pair, float x) {
-    if constexpr (kF16) return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pair), f16x2{0, 0}, x, false);
-    else return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), bf16x2{0, 0}, x, false);
-}
 
 // Eight values of a row as loaded (fp32: two registers of four; 16-bit: one).
 template <typename T> struct Raw { u32x4 v[sizeof(T) == 4 ? 2 : 1]; };

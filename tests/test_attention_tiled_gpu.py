@@ -97,6 +97,30 @@ def test_tiled_values_planes_cannot_carry(dtype, where, value):
     torch.testing.assert_close(got, ref, rtol=2.0 ** -7 if dtype == "bf16" else 2e-3, atol=1e-3, equal_nan=True)
 
 
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.402e38])
+@pytest.mark.parametrize("dim", [3, 300])  # either half of the output's dims
+def test_d512_values_planes_cannot_carry(where, value, dim):
+    S = 70
+    q, k, v = tensors(17, 1, 1, S, 100, 512, "f32")
+    {"q": q, "k": k, "v": v}[where][0, 57, dim] = value
+    got = sh.attention(q, k, v, 1)
+    ref = sh.attention(q, k, v, 1, backend=sh.WARP_ONLINE)
+    if where == "q" and value != value:
+        assert got[0, 57].isnan().all()  # the per-row kernel takes such a row's keys for hidden
+        got[0, 57] = ref[0, 57]
+    torch.testing.assert_close(got, ref, rtol=2e-3, atol=1e-3, equal_nan=True)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk", [
+    (1, 1, 33, 1), (1, 2, 64, 31), (2, 1, 100, 32), (1, 1, 130, 33), (1, 1, 65, 64), (1, 1, 1, 65), (1, 2, 40, 97),
+    (1, 9, 950, 70),   # 270 blocks of 32 queries on 256 CUs: 64 queries per workgroup
+    (1, 6, 1000, 70)])  # 192: 32 queries, all output dims
+def test_d512_blocks(B, H, Sq, Sk):
+    q, k, v = tensors(Sq + Sk, B, H, Sq, Sk, 512, "f32")
+    check(sh.attention(q, k, v, H), reference(q, k, v, H), "f32")
+
+
 def test_tiled_large_logits():
     """Logits of a few hundred, rising along the keys: the running maximum moves in every sub-tile."""
     B, H, S, D = 1, 2, 300, 64
