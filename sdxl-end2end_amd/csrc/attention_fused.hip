@@ -195,8 +195,12 @@ static_assert(2 * 34 * 64 * 4 + 2 * 32 * kRowBytes <= (kKRing + kVRing) * kTileB
 static_assert(4 * 32 * kRowBytes <= (kKRing + kVRing) * kTileBytes, "whole epilogue staging");
 static_assert(2 * 34 * 64 * 4 + (kMixedFull + 2) * 32 * kRowBytes <= 2 * (kKRing + kVRing) * kTileBytes, "mixed epilogue staging");
 
-// The kernel body for one workgroup kind.
-template <int kWaves, bool IsBf16, bool kMaskAll, int kKind>
+// Modes of a group step.
+constexpr int kPlain = 0, kFirst = 1, kHide = 2, kLast = 3;
+
+// The kernel body for one workgroup kind. kTail: k_seq need not fill the last
+// tile or stage (key-split and mixed kinds; the whole kind always handles it).
+template <int kWaves, bool IsBf16, bool kMaskAll, int kKind, bool kTail>
 __device__ __attribute__((always_inline)) inline void attention_body(const FusedAttentionParams& p,
                                                                      char (*ring)[kTileBytes]) {
     constexpr bool split2 = kKind == kKindSplit2;
@@ -234,7 +238,7 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         const int id = split ? (int)blockIdx.x - p.whole_units : (int)blockIdx.x;
         const int xcd = id & 7, slot = id >> 3;
         const int per = n >> 3, extra = n & 7;
-        task = xcd * per + (xcd < extra ? xcd : extra) + slot;
+        task = kMaskAll ? id : xcd * per + (xcd < extra ? xcd : extra) + slot;
     }
     int khalf = split ? wave >> 1 : 0;  // key half (split) or key group (mixed half waves)
     bool half_wave = split;             // one 32-key group per tile step
@@ -254,16 +258,31 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         bh_set[1] = min(first + kMixedBlocks - 1, p.mixed_total - 1) / p.q_blocks;
         nsets = bh_set[1] != bh_set[0] ? 2 : 1;
         set = bh == bh_set[0] ? 0 : 1;
+    } else if constexpr (kMaskAll) {
+        // Masked calls (one kind per launch): the same query block of all heads
+        // together, blocks ranked by the work that a causal limit leaves them
+        // (most first) and dealt to the CUs back and forth: a CU takes
+        // workgroups x, x + CUs, ..., so every odd round of rank_group ranks
+        // runs the other way.
+        const int n_heads = p.batch * p.heads, n_blocks = split ? 2 * p.q_blocks : p.q_blocks;
+        int rank = task / n_heads;
+        bh = task % n_heads;
+        const int first = rank / p.rank_group * p.rank_group;
+        if ((rank / p.rank_group) & 1) rank = first + min(first + p.rank_group, n_blocks) - 1 - rank;
+        const int blk = n_blocks - 1 - rank;
+        q0 = split ? blk * 64 + (wave & 1) * 32 : blk * kBlockQueries + wave * 32;
     } else if constexpr (!split) {
         bh = task / p.q_blocks;
         q0 = (task % p.q_blocks) * kBlockQueries + wave * 32;
     } else {
-        const int blocks64 = p.q_seq / 64;  // q_seq % 128 == 0 for key-split calls
+        const int blocks64 = 2 * p.q_blocks;  // q_blocks: 128-row units per head
         const int gb = 2 * p.whole_units + task;
         bh = gb / blocks64;
         q0 = (gb % blocks64) * 64 + (wave & 1) * 32;
     }
-    const int qblk = q0 / kBlockQueries;
+    // the second half of a head's last unit may lie past its rows
+    if constexpr (split)
+        if ((q0 & ~63) >= p.q_seq) return;
     char (*kring)[kTileBytes] = ring + (mixed ? 4 * set : 0);
     char (*vring)[kTileBytes] = kring + kKRing;
     const int h = bh % p.heads;
@@ -296,18 +315,37 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     // Key range. Causal: keys beyond the block's last query are never visible.
     int n_keys = p.k_seq;
     if (p.causal) {
-        const int last_query = qblk * kBlockQueries + kBlockQueries - 1;
+        const int last_query = (q0 | (split ? 63 : kBlockQueries - 1));
         n_keys = n_keys < last_query + 1 ? n_keys : last_query + 1;
     }
+    // Keys past the last visible one (padding) are not walked: the mask row is
+    // read backwards, 256 keys at a time, up to its last nonzero word.
+    if (kMaskAll && p.key_mask != nullptr) {
+        const int32_t* row = p.key_mask + (int64_t)b * p.k_seq;
+        bool found = false;
+        while (n_keys > 0 && !found) {
+            const int first = n_keys > 256 ? n_keys - 256 : 0;
+            int word[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) word[i] = first + 64 * i + lane < n_keys ? row[first + 64 * i + lane] : 0;
+            int end = first;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint64_t seen = __builtin_amdgcn_ballot_w64(word[i] != 0);
+                if (seen != 0) end = first + 64 * i + 64 - __builtin_clzll(seen);
+            }
+            found = end > first;
+            n_keys = end;
+        }
+    }
     // Key-split calls: stage t holds keys 32t .. +31 of each half (rows 0-31
-    // half 0, rows 32-63 half 1); k_seq % 64 == 0.
-    const int half_keys = p.k_seq / 2;
-    const int n_tiles = split2 ? p.k_seq / (2 * kKeyTile)
-                               : (split || mixed) ? p.k_seq / kKeyTile : (n_keys + kKeyTile - 1) / kKeyTile;
-    // Tiles [0, n_plain) are complete and need no mask (kMaskAll covers key-mask
-    // and causal calls, where every tile is masked).
-    const int n_plain = kMaskAll ? 0 : n_keys / kKeyTile;
-
+    // half 0, rows 32-63 half 1; split2: 64 and rows 64-127). The halves are
+    // whole 32-key (64-key) groups, half 0 the smaller by at most one: only the
+    // last stage can lack keys of either half.
+    const int key_groups = split2 ? (n_keys + kKeyTile - 1) / kKeyTile : (n_keys + 31) / 32;
+    const int half_keys = (split2 ? kKeyTile : 32) * (key_groups >> 1);
+    const int n_tiles = split ? (key_groups + 1) >> 1 : (n_keys + kKeyTile - 1) / kKeyTile;
+    const int key_end = split && khalf == 0 ? half_keys : n_keys;  // of this wave's part
     // ---- tile transfers: the 16 1-KiB transfers of a K tile plus a V tile are
     // split over the waves; transfer n covers the 8-row slab n%8 (rows
     // 8*(n%8) .. +7) of K (n < 8) or V (n >= 8); lane l takes slab row l/8 and
@@ -355,6 +393,17 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         }
     };
 
+    // One slab of a part that k_seq does not fill: rows row0 .. +7 of the part
+    // from key0, into rows lds_row .. +7 of buf; rows past the end re-read the
+    // last key (hidden by the visibility words).
+    auto tail_slab = [&](const char* base, int64_t stride, int key0, int row0, int lds_row, const char* buf) __attribute__((always_inline)) {
+        const int first = min(key0, p.k_seq - 1);
+        const int row = min(row0 + (lane >> 3), p.k_seq - 1 - first);
+        const uint32_t off = __umul24((uint32_t)row, (uint32_t)stride) +
+                             (uint32_t)(((lane & 7) ^ swz(lds_row + (lane >> 3))) << 4);
+        lds_dma16(base + (int64_t)first * stride, off, lds_addr(buf + lds_row * kRowBytes));
+    };
+
     // Key-split stages: slab s covers 8 rows of one key half (slabs 0-3 half
     // 0, 4-7 half 1); stage t holds keys 32t .. +31 of each half.
     auto issue_split = [&](int kt, int vt) __attribute__((always_inline)) {
@@ -365,9 +414,13 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
 #pragma unroll
         for (int j = 0; j < kLoadsPerWave; ++j) {
             const int slab = 2 * j + (wave & 1), half = slab >> 2;
-            const char* slab_base =
-                (is_v ? vbase : kbase) + (int64_t)(half * half_keys + 32 * tile + 8 * (slab & 3)) * whole_stride;
-            lds_dma16(slab_base, whole_off, lds_addr(buf + 8 * slab * kRowBytes));
+            const int key0 = half * half_keys + 32 * tile;
+            if (!(kTail || kMaskAll) || key0 + 32 <= p.k_seq) {
+                const char* slab_base = (is_v ? vbase : kbase) + (int64_t)(key0 + 8 * (slab & 3)) * whole_stride;
+                lds_dma16(slab_base, whole_off, lds_addr(buf + 8 * slab * kRowBytes));
+            } else {
+                tail_slab(is_v ? vbase : kbase, whole_stride, key0, 8 * (slab & 3), 8 * slab, buf);
+            }
         }
     };
 
@@ -384,9 +437,13 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
 #pragma unroll
         for (int j = 0; j < 2 * kLoadsPerWave; ++j) {
             const int slab = 2 * j + (wave & 1), half = slab >> 3;
-            const char* slab_base =
-                (is_v ? vbase : kbase) + (int64_t)(half * half_keys + 64 * tile + 8 * (slab & 7)) * whole_stride;
-            lds_dma16(slab_base, whole_off, lds_addr(buf + 8 * slab * kRowBytes));
+            const int key0 = half * half_keys + 64 * tile;
+            if (!kTail || key0 + 64 <= p.k_seq) {
+                const char* slab_base = (is_v ? vbase : kbase) + (int64_t)(key0 + 8 * (slab & 7)) * whole_stride;
+                lds_dma16(slab_base, whole_off, lds_addr(buf + 8 * slab * kRowBytes));
+            } else {
+                tail_slab(is_v ? vbase : kbase, whole_stride, key0, 8 * (slab & 7), 8 * slab, buf);
+            }
         }
     };
 
@@ -418,6 +475,12 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     const bool mixed_v = wave < kMixedFull;
     const int64_t mixed_stride = mixed_v ? vs_bytes : ks_bytes;
     const uint32_t mixed_off = mixed ? lane_off(wave & 1, mixed_stride) : 0u;
+    auto mixed_slab = [&](const char* base, int64_t stride, int tile, int slab, const char* buf) __attribute__((always_inline)) {
+        if (!kTail || tile * kKeyTile + kKeyTile <= p.k_seq)
+            lds_dma16(base + (int64_t)(tile * kKeyTile + 8 * slab) * stride, mixed_off, lds_addr(buf + 8 * slab * kRowBytes));
+        else
+            tail_slab(base, stride, tile * kKeyTile, 8 * slab, 8 * slab, buf);
+    };
     auto issue_mixed = [&](int kt, int vt) __attribute__((always_inline)) {
         const int tile = mixed_v ? vt : kt;
         if constexpr (!v1_on_half) {
@@ -431,8 +494,7 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
                 for (int j = 0; j < 2; ++j) {
                     if (j == 1 && mixed_v) break;
                     const int slab = mixed_v ? wave : (wave - kMixedFull) + 4 * j;
-                    const char* slab_base = base + (int64_t)(tile * kKeyTile + 8 * slab) * mixed_stride;
-                    lds_dma16(slab_base, mixed_off, lds_addr(buf + 8 * slab * kRowBytes));
+                    mixed_slab(base, mixed_stride, tile, slab, buf);
                 }
             }
         } else {
@@ -446,8 +508,7 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
                     for (int j = 0; j < 2; ++j) {
                         if (j == 1 && mixed_v) break;
                         const int slab = mixed_v ? wave : (wave - kMixedFull) + 4 * j;
-                        const char* slab_base = base + (int64_t)(tile * kKeyTile + 8 * slab) * mixed_stride;
-                        lds_dma16(slab_base, mixed_off, lds_addr(buf + 8 * slab * kRowBytes));
+                        mixed_slab(base, mixed_stride, tile, slab, buf);
                     }
                 }
             }
@@ -457,8 +518,7 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     const int slab = (i & 1) + 4 * (i >> 1) + 2 * j;
-                    const char* slab_base = set_v1 + (int64_t)(vt * kKeyTile + 8 * slab) * vs_bytes;
-                    lds_dma16(slab_base, mixed_off, lds_addr(buf + 8 * slab * kRowBytes));
+                    mixed_slab(set_v1, vs_bytes, vt, slab, buf);
                 }
             }
         }
@@ -548,7 +608,7 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         return shift;
     };
 
-    // One pipelined group step (32 keys of tile t, group g; s_cur holds its
+    // One pipelined group step (32 keys from key0, group g of its buffers; s_cur holds its
     // exp2 arguments c * S - m, scaled in place during the previous step).
     // Overlapped inside the wave: the next group's QK^T chain (K operands in
     // kop, prefetched one step earlier) runs on the matrix core while this
@@ -558,36 +618,43 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     // VALU work issued between it and its predecessor (in-order issue would
     // otherwise stall the wave on the chain). At the end, the K operands of
     // the group after next (tile buffer kn2, group g2) are prefetched into kop.
-    // kMasked/kExact: exact maximum over the whole group first (masked tiles,
-    // first tile); otherwise each half is checked for overflow after the fact.
-    auto group_step = [&]<bool kMasked, bool kExact, bool kPrefetchK = true>(f32x16& s_cur, f32x16& s_next, i16x8 (&kop)[4], const char* vb,
-                                                     int g, int t, uint64_t vis, const char* kn2, int g2,
-                                                     bool have_next) __attribute__((always_inline)) {
+    // Modes: kPlain: each half is checked for overflow after the fact; kFirst:
+    // exact maximum over the whole group first (a row's first group); kHide: as
+    // kPlain, unless hide (wave-uniform) is set: then keys outside the
+    // visibility word or the causal limit are hidden and the maximum is exact
+    // (a branch to code out of line, as the anchor update: the steps of ragged
+    // and masked calls keep the plain step's registers); kLast: hide without the
+    // branch.
+    auto group_step = [&]<int kMode, bool kPrefetchK = true>(f32x16& s_cur, f32x16& s_next, i16x8 (&kop)[4], const char* vb,
+                                                     int g, bool hide, int key0, uint64_t vis, const char* kn2, int g2) __attribute__((always_inline)) {
         // V^T operands of both 16-key halves in their own registers; the second
         // half's are read in slot 3, two slots ahead of their MFMAs (read just
         // before them, c3 94.1 -> 93.8 us, c1 17.1 -> 16.9 us)
         i16x8 vop[2], vop1[2];
         load_v(vb, g, 0, vop);
-        if constexpr (kMasked) {
-            const int key0 = t * kKeyTile + 32 * g;
-            const uint32_t lane_vis = (uint32_t)(vis >> (32 * g + 4 * hf));
-            // causal: key key0 + kk + 4hf is visible iff <= my_query
-            const int causal_lim = p.causal ? my_query - key0 - 4 * hf : 0x7FFFFFFF;
+        if constexpr (kMode == kHide || kMode == kLast) {
+            if (kMode == kLast || __builtin_expect(hide, 0)) {
+                const uint32_t lane_vis = (uint32_t)(vis >> (32 * g + 4 * hf));
+                // causal: key key0 + kk + 4hf is visible iff <= my_query
+                const int causal_lim = p.causal ? my_query - key0 - 4 * hf : 0x7FFFFFFF;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int kk = (i >> 2) * 8 + (i & 3);
-                const bool ok = ((lane_vis >> kk) & 1u) && (kk <= causal_lim);
-                s_cur[i] = ok ? s_cur[i] : -__builtin_inff();
+                for (int i = 0; i < 16; ++i) {
+                    const int kk = (i >> 2) * 8 + (i & 3);
+                    const bool ok = ((lane_vis >> kk) & 1u) && (kk <= causal_lim);
+                    s_cur[i] = ok ? s_cur[i] : -__builtin_inff();
+                }
+                const float shift = exact_max(s_cur, 0, 16);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s_cur[i] -= shift;
             }
-        }
-        if constexpr (kMasked || kExact) {
+        } else if constexpr (kMode == kFirst) {
             const float shift = exact_max(s_cur, 0, 16);
 #pragma unroll
             for (int i = 0; i < 16; ++i) s_cur[i] -= shift;
         }
         float e[16];
         uint32_t pk[8];
-        constexpr bool kCheck = !kMasked && !kExact;
+        constexpr bool kCheck = kMode != kFirst && kMode != kLast;
 
         // Eight slots, each one MFMA followed by about its duration (32 cycles)
         // of VALU work that does not depend on it, pinned with scheduling
@@ -676,7 +743,11 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         acc[1] = mfma32<IsBf16>(vop1[1], p1, acc[1]);
 #pragma unroll
         for (int i = 8; i < 16; ++i) s_next[i] *= c;
-        (void)have_next;
+    };
+
+    // Visibility word of a part with n keys left.
+    auto visible_below = [](int n) __attribute__((always_inline)) -> uint64_t {
+        return n >= kKeyTile ? ~0ull : n > 0 ? (1ull << n) - 1ull : 0ull;
     };
 
     // ---- main loop. Step j = 2t + g handles key group g of tile t; it needs
@@ -700,23 +771,46 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         for (int ks = 1; ks < 4; ++ks) sa = mfma32<IsBf16>(kop[ks], qop[ks], sa);
 #pragma unroll
         for (int i = 0; i < 16; ++i) sa[i] *= c;  // exp2 arguments of the first group
-        auto stage = [&]<bool kFirst, bool kOdd>(int t) __attribute__((always_inline)) {
+        int mask_word = 1;
+        auto load_mask = [&](int t) __attribute__((always_inline)) {
+            if (kMaskAll && p.key_mask != nullptr) {
+                const int key = khalf * half_keys + 32 * t + col;
+                mask_word = key < key_end ? p.key_mask[(int64_t)b * p.k_seq + key] : 0;
+            }
+        };
+        load_mask(0);
+        auto stage = [&]<int kMode, bool kOdd>(int t) __attribute__((always_inline)) {
             wait_vmem_all();  // this lane's transfers of K(t+1), V(t) landed
             __syncthreads();  // ... and every lane's; stage t-1 fully consumed
+            const int key0 = khalf * half_keys + 32 * t;
+            uint32_t vis = ~0u;
+            bool hide = false;
+            if constexpr (kMode == kHide) {
+                if (kMaskAll && p.key_mask != nullptr) vis = (uint32_t)__builtin_amdgcn_ballot_w64(mask_word != 0);
+                if (key0 + 32 > key_end) vis = key0 < key_end ? vis & ((1u << (key_end - key0)) - 1u) : 0u;
+                hide = vis != ~0u;
+                // masked calls: also stages on the causal limit, and those
+                // before every row has seen a visible key
+                if constexpr (kMaskAll)
+                    hide = hide || (p.causal && key0 + 31 > q0) || __builtin_amdgcn_ballot_w64(!anchored) != 0;
+            }
+            load_mask(t + 1);
             issue_split(t + 2, t + 1);
             load_k(kring[kOdd ? 0 : 1], khalf, kop);  // K(t+1) (stale past the end, unused)
             const char* v_t = vring[kOdd ? 1 : 0];
-            if constexpr (kOdd) group_step.template operator()<false, kFirst, false>(sb, sa, kop, v_t, khalf, t, ~0ull, v_t, 0, true);
-            else group_step.template operator()<false, kFirst, false>(sa, sb, kop, v_t, khalf, t, ~0ull, v_t, 0, true);
+            const uint64_t word = (uint64_t)vis << (32 * khalf);
+            if constexpr (kOdd) group_step.template operator()<kMode, false>(sb, sa, kop, v_t, khalf, hide, key0, word, v_t, 0);
+            else group_step.template operator()<kMode, false>(sa, sb, kop, v_t, khalf, hide, key0, word, v_t, 0);
         };
+        constexpr int kRest = kTail || kMaskAll ? kHide : kPlain;
         int t = 0;
         if (n_tiles > 0) {
-            stage.template operator()<true, false>(0);
+            stage.template operator()<kMaskAll ? kHide : kFirst, false>(0);
             for (t = 1; t + 1 < n_tiles; t += 2) {
-                stage.template operator()<false, true>(t);
-                stage.template operator()<false, false>(t + 1);
+                stage.template operator()<kRest, true>(t);
+                stage.template operator()<kRest, false>(t + 1);
             }
-            if (t < n_tiles) stage.template operator()<false, true>(t);
+            if (t < n_tiles) stage.template operator()<kRest, true>(t);
         }
     } else if constexpr (split2) {
         // ---- key-split workgroup with 64 keys of each half per stage: each
@@ -735,23 +829,27 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
 #pragma unroll
         for (int i = 0; i < 16; ++i) sa[i] *= c;  // exp2 arguments of the first group
         load_k(&ring[0][0] + hrow, 1, kop);
-        auto stage2 = [&]<bool kFirst, bool kOdd>(int t) __attribute__((always_inline)) {
+        auto stage2 = [&]<int kMode, bool kOdd>(int t) __attribute__((always_inline)) {
             wait_vmem_all();  // this lane's transfers of K(t+1), V(t) landed
             __syncthreads();  // ... and every lane's; stage t-1 fully consumed
             issue_split2(t + 2, t + 1);
+            const int key0 = khalf * half_keys + kKeyTile * t;
+            const uint64_t vis = kMode == kHide ? visible_below(key_end - key0) : ~0ull;
+            const bool hide = vis != ~0ull;
             const char* v_t = &ring[2 * (kKRing + (kOdd ? 1 : 0))][0] + hrow;
             const char* k_t1 = &ring[2 * (kOdd ? 0 : 1)][0] + hrow;
-            group_step.template operator()<false, kFirst>(sa, sb, kop, v_t, 0, t, ~0ull, k_t1, 0, true);
-            group_step.template operator()<false, false>(sb, sa, kop, v_t, 1, t, ~0ull, k_t1, 1, true);
+            group_step.template operator()<kMode>(sa, sb, kop, v_t, 0, hide, key0, vis, k_t1, 0);
+            group_step.template operator()<kMode == kFirst ? kPlain : kMode>(sb, sa, kop, v_t, 1, hide, key0 + 32, vis, k_t1, 1);
         };
+        constexpr int kRest = kTail ? kHide : kPlain;
         int t = 0;
         if (n_tiles > 0) {
-            stage2.template operator()<true, false>(0);
+            stage2.template operator()<kFirst, false>(0);  // ragged calls: at least two stages
             for (t = 1; t + 1 < n_tiles; t += 2) {
-                stage2.template operator()<false, true>(t);
-                stage2.template operator()<false, false>(t + 1);
+                stage2.template operator()<kRest, true>(t);
+                stage2.template operator()<kRest, false>(t + 1);
             }
-            if (t < n_tiles) stage2.template operator()<false, true>(t);
+            if (t < n_tiles) stage2.template operator()<kRest, true>(t);
         }
     } else if constexpr (mixed) {
         // ---- mixed workgroup: whole waves step through both groups of every
@@ -770,41 +868,48 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         if (!half_wave) load_k(kring[0], 1, kop);
         // Whole and half waves run separate loops (same barrier sequence), so
         // each keeps its own register allocation.
-        auto whole_step = [&]<bool kFirst, bool kOdd>(int t) __attribute__((always_inline)) {
+        auto whole_step = [&]<int kMode, bool kOdd>(int t) __attribute__((always_inline)) {
             wait_vmem_all();  // this lane's transfers of K(t+1), V(t) landed
             __syncthreads();  // ... and every lane's; step t-1 fully consumed
             issue_mixed(t + 2, t + 1);
+            const int key0 = t * kKeyTile;
+            const uint64_t vis = kMode == kHide ? visible_below(p.k_seq - key0) : ~0ull;
+            const bool hide = vis != ~0ull;
             const char* v_t = vring[kOdd ? 1 : 0];
             const char* k_t1 = kring[kOdd ? 0 : 1];
-            group_step.template operator()<false, kFirst>(sa, sb, kop, v_t, 0, t, ~0ull, k_t1, 0, true);
-            group_step.template operator()<false, false>(sb, sa, kop, v_t, 1, t, ~0ull, k_t1, 1, true);
+            group_step.template operator()<kMode>(sa, sb, kop, v_t, 0, hide, key0, vis, k_t1, 0);
+            group_step.template operator()<kMode == kFirst ? kPlain : kMode>(sb, sa, kop, v_t, 1, hide, key0 + 32, vis, k_t1, 1);
         };
-        auto half_step = [&]<bool kFirst, bool kOdd>(int t) __attribute__((always_inline)) {
+        auto half_step = [&]<int kMode, bool kOdd>(int t) __attribute__((always_inline)) {
             wait_vmem_all();
             __syncthreads();
             issue_mixed(t + 2, t + 1);
+            const int key0 = t * kKeyTile + 32 * khalf;
+            const uint64_t vis = kMode == kHide ? visible_below(p.k_seq - t * kKeyTile) : ~0ull;
+            const bool hide = vis != ~0ull;
             const char* v_t = vring[kOdd ? 1 : 0];
             load_k(kring[kOdd ? 0 : 1], khalf, kop);  // K(t+1) (stale past the end, unused)
-            if constexpr (kOdd) group_step.template operator()<false, kFirst, false>(sb, sa, kop, v_t, khalf, t, ~0ull, v_t, 0, true);
-            else group_step.template operator()<false, kFirst, false>(sa, sb, kop, v_t, khalf, t, ~0ull, v_t, 0, true);
+            if constexpr (kOdd) group_step.template operator()<kMode, false>(sb, sa, kop, v_t, khalf, hide, key0, vis, v_t, 0);
+            else group_step.template operator()<kMode, false>(sa, sb, kop, v_t, khalf, hide, key0, vis, v_t, 0);
         };
-        // n_tiles >= 1 (k_seq >= 64)
+        // n_tiles >= 1 (k_seq >= 64); ragged calls: at least three
+        constexpr int kRest = kTail ? kHide : kPlain;
         if (!half_wave) {
-            whole_step.template operator()<true, false>(0);
+            whole_step.template operator()<kFirst, false>(0);
             int t = 1;
             for (; t + 1 < n_tiles; t += 2) {
-                whole_step.template operator()<false, true>(t);
-                whole_step.template operator()<false, false>(t + 1);
+                whole_step.template operator()<kRest, true>(t);
+                whole_step.template operator()<kRest, false>(t + 1);
             }
-            if (t < n_tiles) whole_step.template operator()<false, true>(t);
+            if (t < n_tiles) whole_step.template operator()<kRest, true>(t);
         } else {
-            half_step.template operator()<true, false>(0);
+            half_step.template operator()<kFirst, false>(0);
             int t = 1;
             for (; t + 1 < n_tiles; t += 2) {
-                half_step.template operator()<false, true>(t);
-                half_step.template operator()<false, false>(t + 1);
+                half_step.template operator()<kRest, true>(t);
+                half_step.template operator()<kRest, false>(t + 1);
             }
-            if (t < n_tiles) half_step.template operator()<false, true>(t);
+            if (t < n_tiles) half_step.template operator()<kRest, true>(t);
         }
     } else {
     if (n_tiles > 0) {
@@ -822,45 +927,74 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     }
     // kOdd: parity of t, so that every ring slot below is a compile-time
     // offset (folded into the LDS instructions' immediates).
-    auto tile = [&]<bool kMasked, bool kFirst, bool kOdd>(int t) __attribute__((always_inline)) {
+    int mask_word = 1;
+    auto load_mask = [&](int t) __attribute__((always_inline)) {
+        if (kMaskAll && p.key_mask != nullptr) {
+            const int key = t * kKeyTile + lane;
+            mask_word = key < p.k_seq ? p.key_mask[(int64_t)b * p.k_seq + key] : 0;
+        }
+    };
+    if (n_tiles > 0) load_mask(0);
+    auto tile = [&]<int kMode, bool kOdd>(int t) __attribute__((always_inline)) {
         wait_vmem_all();  // this lane's transfers of K(t+1), V(t) landed
         __syncthreads();  // ... and every lane's; tile t-1 fully consumed
+        const int key0 = t * kKeyTile;
         uint64_t vis = ~0ull;
-        if constexpr (kMasked) {
-            // vis bit j: key 64t + j exists and is not masked out (wave-uniform).
-            const int key0 = t * kKeyTile;
-            if (p.key_mask != nullptr) {
-                const int key = key0 + lane;
-                const int word = key < p.k_seq ? p.key_mask[(int64_t)b * p.k_seq + key] : 0;
-                vis = __builtin_amdgcn_ballot_w64(word != 0);
-            }
-            if (key0 + kKeyTile > p.k_seq) vis &= (1ull << (p.k_seq - key0)) - 1ull;
+        if constexpr (kMode == kHide || kMode == kLast) {
+            // bit j: key 64t + j exists and is not masked out (wave-uniform)
+            if (kMaskAll && p.key_mask != nullptr) vis = __builtin_amdgcn_ballot_w64(mask_word != 0);
+            vis &= visible_below(p.k_seq - key0);
         }
+        load_mask(t + 1);
         issue(t + 2, t + 1);
         const char* v_t = vring[kOdd ? 1 : 0];
         const char* k_t1 = kring[kOdd ? 0 : 1];
-        group_step.template operator()<kMasked, kMasked || kFirst>(sa, sb, kop, v_t, 0, t, vis, k_t1, 0, true);
-        group_step.template operator()<kMasked, kMasked>(sb, sa, kop, v_t, 1, t, vis, k_t1, 1, true);
+        // masked calls: also groups on the causal limit, and those before every
+        // row has seen a visible key
+        auto hide = [&](int g) __attribute__((always_inline)) {
+            bool r = (uint32_t)(vis >> (32 * g)) != ~0u;
+            if constexpr (kMaskAll)
+                r = r || (p.causal && key0 + 32 * g + 31 > q0) || __builtin_amdgcn_ballot_w64(!anchored) != 0;
+            return r;
+        };
+        group_step.template operator()<kMode>(sa, sb, kop, v_t, 0, hide(0), key0, vis, k_t1, 0);
+        group_step.template operator()<kMode == kFirst ? kPlain : kMode>(sb, sa, kop, v_t, 1, hide(1), key0 + 32, vis, k_t1, 1);
     };
+    // Unmasked ragged calls have more than one tile (k_seq > 128): their last
+    // one alone has keys to hide. Masked calls decide for every tile.
     int t = 0;
-    if (n_plain > 0) {
-        tile.template operator()<false, true, false>(0);
-        for (t = 1; t + 1 < n_plain; t += 2) {
-            tile.template operator()<false, false, true>(t);
-            tile.template operator()<false, false, false>(t + 1);
+    if constexpr (kMaskAll) {
+        if (n_tiles > 0) {
+            tile.template operator()<kHide, false>(0);
+            for (t = 1; t + 1 < n_tiles; t += 2) {
+                tile.template operator()<kHide, true>(t);
+                tile.template operator()<kHide, false>(t + 1);
+            }
+            if (t < n_tiles) tile.template operator()<kHide, true>(t);
         }
-        if (t < n_plain) {
-            tile.template operator()<false, false, true>(t);
-            ++t;
+    } else {
+        const int n_full = n_keys / kKeyTile;
+        if (n_full > 0) {
+            tile.template operator()<kFirst, false>(0);
+            for (t = 1; t + 1 < n_full; t += 2) {
+                tile.template operator()<kPlain, true>(t);
+                tile.template operator()<kPlain, false>(t + 1);
+            }
+            if (t < n_full) {
+                tile.template operator()<kPlain, true>(t);
+                ++t;
+            }
         }
-    }
-    if ((t & 1) && t < n_tiles) {
-        tile.template operator()<true, false, true>(t);
-        ++t;
-    }
-    for (; t < n_tiles; t += 2) {
-        tile.template operator()<true, false, false>(t);
-        if (t + 1 < n_tiles) tile.template operator()<true, false, true>(t + 1);
+        if constexpr (kTail) {
+            if ((t & 1) && t < n_tiles) {
+                tile.template operator()<kLast, true>(t);
+                ++t;
+            }
+            for (; t < n_tiles; t += 2) {
+                tile.template operator()<kLast, false>(t);
+                if (t + 1 < n_tiles) tile.template operator()<kLast, true>(t + 1);
+            }
+        }
     }
 
     }  // whole workgroup
@@ -930,40 +1064,44 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     }
 }
 
+// Ragged and masked calls (kTail, kMaskAll) decide per group, by a wave-uniform
+// branch, whether keys have to be hidden, so that their other groups take the
+// plain step: masked causal fp16 [2, 16, 1500] 47.6 us with every group masked
+// on whole workgroups, 31.7 with the branch, key-split workgroups and the
+// ranked order; fp16 [2, 10, 3952], ragged, 103 us on whole workgroups alone,
+// 90 on the mixed kind.
 // Whole and key-split workgroups share one kernel (one grid); each kind is
 // a separate instantiation of the body, so neither constrains the other's
 // register allocation. K ring then V ring in one array (the key-split merge
 // reuses all of it).
-template <int kWaves, bool IsBf16, bool kMaskAll>
+template <int kWaves, bool IsBf16, bool kMaskAll, bool kTail>
 __global__ __launch_bounds__(kWaves * 64, 3) void fused_attention_d64_kernel(FusedAttentionParams p) {
     __shared__ __attribute__((aligned(16))) char ring[kKRing + kVRing][kTileBytes];
-    if constexpr (!kMaskAll) {
-        if ((int)blockIdx.x >= p.whole_units) {
-            attention_body<kWaves, IsBf16, false, kKindSplit>(p, ring);
-            return;
-        }
+    if ((int)blockIdx.x >= p.whole_units) {
+        attention_body<kWaves, IsBf16, kMaskAll, kKindSplit, kTail>(p, ring);
+        return;
     }
-    attention_body<kWaves, IsBf16, kMaskAll, kKindWhole>(p, ring);
+    attention_body<kWaves, IsBf16, kMaskAll, kKindWhole, kTail>(p, ring);
 }
 
 // Whole workgroups with split2 key-split ones (64 KiB of LDS: two per CU),
 // for single-round grids of at most two workgroups per CU.
-template <bool IsBf16>
+template <bool IsBf16, bool kTail>
 __global__ __launch_bounds__(4 * 64, 2) void fused_attention_d64_wide_kernel(FusedAttentionParams p) {
     __shared__ __attribute__((aligned(16))) char ring[2 * (kKRing + kVRing)][kTileBytes];
     if ((int)blockIdx.x >= p.whole_units) {
-        attention_body<4, IsBf16, false, kKindSplit2>(p, ring);
+        attention_body<4, IsBf16, false, kKindSplit2, kTail>(p, ring);
         return;
     }
-    attention_body<4, IsBf16, false, kKindWhole>(p, ring);
+    attention_body<4, IsBf16, false, kKindWhole, kTail>(p, ring);
 }
 
 // Mixed workgroups: 12 waves, one workgroup per CU; K and V rings for up to
 // two heads (the key-part merge reuses the first of them).
-template <bool IsBf16, int kKind = kKindMixed>
+template <bool IsBf16, int kKind, bool kTail>
 __global__ __launch_bounds__(12 * 64, 3) void fused_attention_d64_mixed_kernel(FusedAttentionParams p) {
     __shared__ __attribute__((aligned(16))) char ring[2 * (kKRing + kVRing)][kTileBytes];
-    attention_body<12, IsBf16, false, kKind>(p, ring);
+    attention_body<12, IsBf16, false, kKind, kTail>(p, ring);
 }
 
 // ---- short key sequences (k_seq <= 128: the 77-token cross-attention, CLIP).
@@ -1554,15 +1692,15 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
     // key-split workgroups (64 rows, each wave half the keys: half the work of
     // a whole one), see below.
     // The hardware deals ids x, x + CUs, x + 2 CUs to one CU, so with whole
-    // workgroups first every CU of the last round gets the same mix.
-    // Non-causal, unmasked calls with q_seq % 128 == 0 and k_seq % 64 == 0.
+    // workgroups first every CU of the last round gets the same mix. Unmasked
+    // calls; lengths that do not fill the last stage run the kTail forms.
     p.whole_units = p.total_blocks;
     p.split_units = 0;
     bool wide = false;  // whole + split2 workgroups on the 64-KiB kernel
     const int64_t slots = (int64_t)compute_units * 3;
     const int64_t units = p.total_blocks;
-    if (compute_units > 0 && !p.causal && p.key_mask == nullptr && p.q_seq % 128 == 0 && p.k_seq % 64 == 0 &&
-        p.k_seq > 0 && units % slots != 0) {
+    const bool mask_all = p.causal || p.key_mask != nullptr;
+    if (compute_units > 0 && !mask_all && p.k_seq > 0 && units % slots != 0) {
         const int64_t full = units - units % slots, rem = units % slots;
         // Whole workgroups do more per transfer and per barrier than two
         // key-split ones (two groups per tile step, one staging per 4 blocks):
@@ -1578,7 +1716,7 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
             p.split_units = (int32_t)(2 * r);
             // one round of at most two workgroups per CU: key-split workgroups
             // with 64 keys of each half per stage
-            wide = full == 0 && q == 1 && 2 * r <= compute_units && p.k_seq % 128 == 0;
+            wide = full == 0 && q == 1 && 2 * r <= compute_units;
         } else if (2 * rem >= slots) {
             p.whole_units = (int32_t)(full + 2 * rem - slots);
             p.split_units = (int32_t)(2 * slots - 2 * rem);
@@ -1587,17 +1725,32 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
             p.split_units = (int32_t)(2 * rem);
             // one round of at most two key-split workgroups per CU: the 64-KiB
             // kind too ([1,10,1024,1024] 11.5 -> 10.9 us)
-            wide = full == 0 && rem <= compute_units && p.k_seq % 128 == 0;
+            wide = full == 0 && rem <= compute_units;
         }
     }
-    const bool mask_all = p.causal || p.key_mask != nullptr;
+    // Ragged calls (their last stage holds hidden keys, and a unit may hold 64
+    // empty rows) take the key-split workgroups only where they relieve the
+    // most-loaded CU (workgroups x, x + CUs, ... share one) and the sequence is
+    // long enough for the merge: bf16 [2, 20, 988] 23.0 -> 21.5 us, [1, 20, 500]
+    // 10.1 -> 9.8; without the rule [2, 20, 300] 8.7 -> 9.4, [4, 20, 700]
+    // 21.5 -> 22.1.
+    if (p.split_units > 0 && (p.q_seq % 128 != 0 || p.k_seq % 64 != 0)) {
+        auto per_cu = [&](int64_t n) { return (n + compute_units - 1) / compute_units; };
+        const int64_t cut = per_cu(p.whole_units) + per_cu((int64_t)p.whole_units + p.split_units);  // in half units
+        if (cut >= 2 * per_cu(units) || p.k_seq < 448) {
+            p.whole_units = (int32_t)units;
+            p.split_units = 0;
+            wide = false;
+        }
+    }
     // Mixed 12-wave workgroups (10 row blocks each, one per CU at a time) when
     // their rounds carry at most 10% more blocks per CU than an even share:
     // per SIMD 2.5 blocks with one K/V staging per 10 blocks. Measured against
     // the 4-wave grids in one process: [2,10,4096] 92.5 vs 94.0 us (exact
     // fit), [4,20,960] 26.5 vs 29.5 us (240 of 256 CUs busy), [4,10,3840]
     // 157.9 vs 169.9 us (two rounds, 480 workgroups).
-    if (compute_units > 0 && !mask_all && p.k_seq % 64 == 0 && p.k_seq > 0) {
+    const bool tail64 = p.k_seq % 64 != 0, tail128 = p.k_seq % 128 != 0;
+    if (compute_units > 0 && !mask_all && p.k_seq > 0) {
         const int64_t qb32 = (p.q_seq + 31) / 32;
         const int64_t total = qb32 * p.heads * p.batch;
         const int64_t wgs = (total + kMixedBlocks - 1) / kMixedBlocks;
@@ -1612,28 +1765,48 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
             // waves' V transfers reuse their K offsets)
             const bool spans = qb32 % kMixedBlocks != 0 && p.heads * p.batch > 1 && p.k_row_stride == p.v_row_stride;
             const dim3 g(p.mixed_wgs), b(768);
-            if (spans) {
-                if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_mixed_kernel<true, kKindMixed2>), g, b, 0, stream, p);
-                else hipLaunchKernelGGL((fused_attention_d64_mixed_kernel<false, kKindMixed2>), g, b, 0, stream, p);
-            } else {
-                if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_mixed_kernel<true>), g, b, 0, stream, p);
-                else hipLaunchKernelGGL((fused_attention_d64_mixed_kernel<false>), g, b, 0, stream, p);
-            }
+#define SDXL_MIXED(BF, KIND)                                                                                     \
+    do {                                                                                                         \
+        if (tail64) hipLaunchKernelGGL((fused_attention_d64_mixed_kernel<BF, KIND, true>), g, b, 0, stream, p);  \
+        else hipLaunchKernelGGL((fused_attention_d64_mixed_kernel<BF, KIND, false>), g, b, 0, stream, p);        \
+    } while (0)
+            if (spans && is_bf16) SDXL_MIXED(true, kKindMixed2);
+            else if (spans) SDXL_MIXED(false, kKindMixed2);
+            else if (is_bf16) SDXL_MIXED(true, kKindMixed);
+            else SDXL_MIXED(false, kKindMixed);
+#undef SDXL_MIXED
             return hipGetLastError();
         }
     }
-    const dim3 grid(p.whole_units + p.split_units), block(64 * kFusedWaves);
-    if (wide) {
-        if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((fused_attention_d64_wide_kernel<false>), grid, block, 0, stream, p);
-        return hipGetLastError();
+    if (mask_all) {
+        // Masked calls, one kind per launch: key-split workgroups (64 rows)
+        // while they all fit three per CU under a causal limit, whose blocks
+        // are of unequal length, and while whole ones would not fill two per CU
+        // without it; else whole ones. Measured, split against whole: causal
+        // [2, 16, 1500] 23.4 / 29.3 us, [4, 20, 1000] 30.7 / 31.3, [4, 20, 2000]
+        // (1280 units) 75.7 / 72.4; key mask alone [2, 16, 1500] 43 / 50,
+        // [4, 20, 1000] (640 units) 51.5 / 43.9.
+        if (units <= (p.causal ? slots : 2 * (int64_t)compute_units - 1)) {
+            p.whole_units = 0;
+            p.split_units = (int32_t)(2 * units);
+        }
+        const int64_t heads_total = (int64_t)p.heads * p.batch;
+        p.rank_group = compute_units > heads_total ? (int32_t)(compute_units / heads_total) : 1;
     }
-    if (is_bf16) {
-        if (mask_all) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, true, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, true, false>), grid, block, 0, stream, p);
+    const dim3 grid(p.whole_units + p.split_units), block(64 * kFusedWaves);
+    if (mask_all) {
+        if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, true, true, false>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, false, true, false>), grid, block, 0, stream, p);
+    } else if (wide) {
+        if (is_bf16 && tail128) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<true, true>), grid, block, 0, stream, p);
+        else if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<true, false>), grid, block, 0, stream, p);
+        else if (tail128) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<false, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((fused_attention_d64_wide_kernel<false, false>), grid, block, 0, stream, p);
     } else {
-        if (mask_all) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, false, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, false, false>), grid, block, 0, stream, p);
+        if (is_bf16 && tail64) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, true, false, true>), grid, block, 0, stream, p);
+        else if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, true, false, false>), grid, block, 0, stream, p);
+        else if (tail64) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, false, false, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, false, false, false>), grid, block, 0, stream, p);
     }
     return hipGetLastError();
 }

@@ -1,0 +1,89 @@
+"""Ragged and masked 16-bit head_dim-64 calls on every workgroup kind, against 64-bit attention: key
+counts around the edges of the last stage, query counts that leave half a unit empty, key masks with
+hidden ends, and the anchor update in the groups that ragged calls branch around."""
+import pytest
+
+import sdxl_hip as sh
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+DTYPES = {"f16": torch.float16, "bf16": torch.bfloat16}
+# Rounding of the probabilities and of the output (unit roundoff 2^-11, 2^-8): |error| <= 2 u sum_j
+# p_j |v_j| <= 2 u max |v| at worst, far less where the probabilities spread; max |v| < 5.5.
+UNIT = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+
+
+def tensors(seed, B, H, Sq, Sk, dtype, q_scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    make = lambda s, c=1.0: (torch.randn(B, s, H * 64, device=DEV, generator=g) * c).to(DTYPES[dtype])
+    return make(Sq, q_scale), make(Sk), make(Sk)
+
+
+def check(q, k, v, H, dtype, causal=False, key_mask=None, rows=None):
+    got = sh.attention(q, k, v, H, causal=causal, key_mask=key_mask)
+    B, Sq, _ = q.shape
+    Sk = k.shape[1]
+    worst = 0.0
+    for b in range(B):
+        for h in range(H):
+            c = slice(h * 64, (h + 1) * 64)
+            s = q[b, :, c].double() @ k[b, :, c].double().t() / 8
+            if key_mask is not None:
+                s.masked_fill_(key_mask[b][None] == 0, float("-inf"))
+            if causal:
+                s.masked_fill_(torch.ones(Sq, Sk, dtype=torch.bool, device=DEV).triu(1), float("-inf"))
+            p = torch.nan_to_num(torch.softmax(s, -1))
+            ref = p @ v[b, :, c].double()
+            bound = 2 * UNIT[dtype] * (p @ v[b, :, c].double().abs()) + 1e-6
+            worst = max(worst, ((got[b, :, c].double() - ref).abs() / bound).max().item())
+    assert worst <= 1.0, worst
+    return got
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("B,H,Sq,Sk", [
+    # key-split workgroups on the 64-KiB kernel, alone and beside whole ones
+    (1, 2, 450, 449), (1, 2, 512, 511), (1, 3, 321, 480), (1, 2, 640, 545), (1, 2, 200, 576), (2, 20, 988, 988),
+    # ... on the 32-KiB kernel (three workgroups per CU)
+    (1, 75, 700, 450), (1, 75, 700, 481), (1, 75, 700, 512),
+    # mixed workgroups within one head (blocks a multiple of 10 per head) and across two
+    (2, 16, 2560, 129), (4, 8, 2559, 191), (2, 10, 4090, 160), (4, 20, 930, 223), (4, 20, 930, 1000),
+    # whole workgroups
+    (2, 20, 300, 300), (1, 2, 130, 129)])
+def test_ragged(B, H, Sq, Sk, dtype):
+    check(*tensors(Sq + Sk, B, H, Sq, Sk, dtype), H, dtype)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("B,H,Sq,Sk", [
+    (2, 3, 150, 170), (3, 2, 333, 500), (2, 2, 700, 300), (1, 5, 257, 1025),
+    (2, 256, 200, 190)])  # whole workgroups: more units than key-split ones are used for
+def test_masked(B, H, Sq, Sk, causal, dtype):
+    q, k, v = tensors(Sq + Sk, B, H, Sq, Sk, dtype)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    if causal:
+        check(q, k, v, H, dtype, causal=True)
+    kept = torch.zeros(B, Sk, dtype=torch.int32, device=DEV)
+    kept[0, 40: Sk - 70] = 1                                  # hidden at both ends
+    if B > 1:
+        kept[1] = (torch.rand(Sk, device=DEV, generator=g) < 0.5).int()
+    got = check(q, k, v, H, dtype, causal=causal, key_mask=kept)
+    if B > 2:
+        assert (got[2] == 0).all()                            # nothing visible
+    one = torch.zeros(B, Sk, dtype=torch.int32, device=DEV)
+    one[:, Sk // 2] = -7                                      # any nonzero word shows its key
+    check(q, k, v, H, dtype, causal=causal, key_mask=one)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 2, 450, 449), (1, 75, 700, 450), (4, 20, 930, 223), (2, 20, 300, 300)])
+def test_ragged_anchor_update(B, H, Sq, Sk):
+    """A key far above the rest in a middle group, in the last complete one and in the ragged one."""
+    for at in (Sk // 2, Sk // 32 * 32 - 5, Sk - 1):
+        q, k, v = tensors(at, B, H, Sq, Sk, "f16", q_scale=4.0)
+        k[:, at] = 3 * q.mean(dim=1)
+        k[:, at] += k[:, at].sign() * 4
+        check(q, k, v, H, "f16")
+        check(q, k, v, H, "f16", causal=True)
