@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.environ.get("SDXL_HIP_LIB") or os.path.join(PKG_ROOT, "lib", "libsdxl_attn.so")
@@ -90,6 +91,16 @@ class CrossSublayerDesc(ctypes.Structure):
                 ("ln_eps", ctypes.c_float), ("q_activations", ctypes.c_int32)]
 
 
+# The descriptors as packed bytes (native alignment, as the structures above) and prototypes that
+# take them: on the call path one struct.pack costs a third of filling a ctypes structure.
+_ATTN_DESC = struct.Struct("9q4if4x")
+_LINEAR_DESC = struct.Struct("7q2i")
+_SUBLAYER_DESC = struct.Struct("3q2if2i4x")
+_CROSS_SUBLAYER_DESC = struct.Struct("4q2ifi")
+assert _ATTN_DESC.size == ctypes.sizeof(AttnDesc) and _LINEAR_DESC.size == ctypes.sizeof(LinearDesc)
+assert _SUBLAYER_DESC.size == ctypes.sizeof(SublayerDesc) and _CROSS_SUBLAYER_DESC.size == ctypes.sizeof(CrossSublayerDesc)
+
+
 class SdxlError(RuntimeError):
     """Raised for a non-OK sdxl_status; mirrors the reference's CudaError."""
 
@@ -156,6 +167,11 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.sdxl_cross_attn_sublayer.restype = ctypes.c_int
     lib.sdxl_cross_attn_sublayer.argtypes = [ctypes.POINTER(CrossSublayerDesc), vp, vp, vp, vp, vp, vp, i64, vp, vp,
                                              vp, vp, ctypes.c_size_t, vp]
+    for name in ("sdxl_attn_fwd", "sdxl_linear", "sdxl_attn_sublayer", "sdxl_cross_attn_sublayer"):
+        fn = lib[name]  # a function object of its own, with its own prototype
+        fn.restype = ctypes.c_int
+        fn.argtypes = [ctypes.c_char_p] + getattr(lib, name).argtypes[1:]
+        setattr(lib, "packed_" + name, fn)
     _LIB = lib
     return lib
 
@@ -197,12 +213,30 @@ def fwd_raw(desc: AttnDesc, q_ptr: int, k_ptr: int, v_ptr: int, mask_ptr: int, o
                                 stream or None))
 
 
-def _dtype_code(t) -> int:
-    import torch
-    m = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
-    if t.dtype not in m:
-        raise SdxlError(INVALID_SHAPE, "CUDA attention mismatch")
-    return m[t.dtype]
+class _Torch:
+    """What the call paths use of torch, looked up once (torch is imported with the first call)."""
+
+    loaded = None
+
+    def __init__(self):
+        import torch
+        self.codes = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
+        self.f16, self.int32, self.uint8 = torch.float16, torch.int32, torch.uint8
+        self.empty, self.empty_like = torch.empty, torch.empty_like
+        # the handle of the current stream without a Stream object around it
+        self.raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+            (lambda index: torch.cuda.current_stream(index).cuda_stream)
+        _Torch.loaded = self
+
+
+def _f32(x) -> float:
+    """x, or the infinity that it rounds to (which the library refuses) where struct would not pack it."""
+    return x if -3.4028234663852886e38 <= x <= 3.4028234663852886e38 else x * float("inf")
+
+
+def _check_packed(status: int) -> None:
+    if status != OK:
+        _check(status)
 
 
 def attention(query, key, value, heads: int, causal: bool = False, key_mask=None,
@@ -213,31 +247,36 @@ def attention(query, key, value, heads: int, causal: bool = False, key_mask=None
     wider when the tensors are column slices of a fused projection). Returns [B, Sq, W].
     Shape checks follow reference src/cuda/ops_kernels.cu:1914-1926.
     """
-    import torch
+    t = _Torch.loaded or _Torch()
     if isinstance(backend, str):
         backend = parse_backend(backend)
-    if (query.dim() != 3 or key.dim() != 3 or value.shape != key.shape or query.dtype != key.dtype
-            or value.dtype != key.dtype or query.shape[0] != key.shape[0]
-            or query.shape[2] != key.shape[2] or heads <= 0 or query.shape[2] % heads != 0):
+    q_shape, k_shape, dtype = query.shape, key.shape, query.dtype
+    if (len(q_shape) != 3 or len(k_shape) != 3 or value.shape != k_shape or dtype != key.dtype or value.dtype != dtype
+            or q_shape[0] != k_shape[0] or q_shape[2] != k_shape[2] or heads <= 0 or q_shape[2] % heads != 0
+            or dtype not in t.codes):
         raise SdxlError(INVALID_SHAPE, "CUDA attention mismatch")
-    for t in (query, key, value):
-        if t.numel() == 0:
-            continue
-        if t.stride(2) != 1 or (t.shape[0] > 1 and t.stride(0) != t.shape[1] * t.stride(1)):
+    B, Sq, W = q_shape
+    Sk = k_shape[1]
+    q_stride, k_stride, v_stride = query.stride(), key.stride(), value.stride()
+    for stride, rows in ((q_stride, Sq), (k_stride, Sk), (v_stride, Sk)):
+        if B * rows * W != 0 and (stride[2] != 1 or (B > 1 and stride[0] != rows * stride[1])):
             raise SdxlError(INVALID_SHAPE, "sdxl_attn: tensors must be row-major [B, S, stride]")
     if key_mask is not None:
-        if (key_mask.dtype != torch.int32 or key_mask.dim() != 2 or key_mask.shape[0] != key.shape[0]
-                or key_mask.shape[1] != key.shape[1] or not key_mask.is_contiguous()):
+        if (key_mask.dtype != t.int32 or key_mask.dim() != 2 or key_mask.shape[0] != B
+                or key_mask.shape[1] != Sk or not key_mask.is_contiguous()):
             raise SdxlError(INVALID_SHAPE, "CUDA attention key mask mismatch")
-    B, Sq, W = query.shape
-    Sk = key.shape[1]
     if out is None:
-        out = torch.empty((B, Sq, W), dtype=query.dtype, device=query.device)
-    desc = make_desc(B, Sq, Sk, heads, W // heads, _dtype_code(query), causal, backend, scale,
-                     (query.stride(1), key.stride(1), value.stride(1), out.stride(1)))
-    stream = torch.cuda.current_stream(query.device).cuda_stream if query.is_cuda else 0
-    fwd_raw(desc, query.data_ptr(), key.data_ptr(), value.data_ptr(),
-            key_mask.data_ptr() if key_mask is not None else 0, out.data_ptr(), stream)
+        out = query.new_empty((B, Sq, W))
+        o_stride = W
+    else:
+        o_stride = out.stride(1)
+    desc = _ATTN_DESC.pack(B, Sq, Sk, heads, W // heads, q_stride[1], k_stride[1], v_stride[1], o_stride,
+                           t.codes[dtype], 1 if causal else 0, backend, 0, _f32(scale))
+    index = query.get_device()
+    _check_packed(load().packed_sdxl_attn_fwd(
+        desc, query.data_ptr(), key.data_ptr(), value.data_ptr(),
+        key_mask.data_ptr() if key_mask is not None else None, out.data_ptr(),
+        t.raw_stream(index) if index >= 0 else None))
     return out
 
 
@@ -309,18 +348,22 @@ def linear_e4m3(a, a_scale, w, w_scale, bias=None, residual=None, out=None):
 def linear(a, w, w_scale=None, bias=None, residual=None, out=None):
     """Ops::linear: a [M, K] fp16, w [N, K] fp16 or uint8 E4M3 codes (with w_scale [N] fp32),
     optional bias [N] and residual [M, N]; returns [M, N] fp16 (2-D views with unit column stride)."""
-    import torch
     M, K = a.shape
-    N = w.shape[0]
     if out is None:
-        out = torch.empty((M, N), dtype=torch.float16, device=a.device)
-    d = LinearDesc(m=M, n=N, k=K, a_row_stride=a.stride(0), w_row_stride=w.stride(0),
-                   c_row_stride=out.stride(0),
-                   residual_row_stride=residual.stride(0) if residual is not None else 0,
-                   w_dtype=E4M3 if w.dtype == torch.uint8 else F16, reserved=0)
-    _check(load().sdxl_linear(ctypes.byref(d), _ptr(a), _ptr(w), _ptr(w_scale), _ptr(bias), _ptr(residual),
-                              _ptr(out), _stream(a)))
+        out = a.new_empty((M, w.shape[0]), dtype=(_Torch.loaded or _Torch()).f16)
+    _linear(M, K, a, a.stride(0), w, w_scale, bias, residual, out, out.stride(0))
     return out
+
+
+def _linear(M, K, a, a_stride, w, w_scale, bias, residual, out, out_stride) -> None:
+    t = _Torch.loaded or _Torch()
+    desc = _LINEAR_DESC.pack(M, w.shape[0], K, a_stride, w.stride(0), out_stride,
+                             residual.stride(0) if residual is not None else 0, E4M3 if w.dtype == t.uint8 else F16, 0)
+    index = a.get_device()
+    _check_packed(load().packed_sdxl_linear(
+        desc, a.data_ptr(), w.data_ptr(), w_scale.data_ptr() if w_scale is not None else None,
+        bias.data_ptr() if bias is not None else None, residual.data_ptr() if residual is not None else None,
+        out.data_ptr(), t.raw_stream(index) if index >= 0 else None))
 
 
 def layer_norm_linear(x, gamma, beta, w, w_scale, bias=None, eps: float = 1e-5, out=None,
@@ -364,19 +407,19 @@ def attn_sublayer(x, ln_gamma, ln_beta, w_qkv, w_qkv_scale, w_out, b_out, heads:
     """x + to_out(attention(LN(x) . w_qkv^T)) for hidden x [B, S, W] fp16 (reference
     src/cuda/unet.cpp:106-118 with q/k/v fused): w_qkv [3W, W] fp16 or uint8 E4M3 + w_qkv_scale [3W].
     fp8_activations: LayerNorm emits E4M3 codes and the QKV projection runs on fp8 MFMA."""
-    import torch
+    t = _Torch.loaded or _Torch()
     B, S, W = x.shape
     if out is None:
-        out = torch.empty_like(x)
-    d = SublayerDesc(batch=B, seq=S, heads=heads, w_qkv_dtype=E4M3 if w_qkv.dtype == torch.uint8 else F16,
-                     attn_backend=backend, ln_eps=eps, qkv_activations=E4M3 if fp8_activations else F16,
-                     ln_fusion=0 if ln_fusion else 1)
-    nbytes = int(load().sdxl_attn_sublayer_workspace_bytes(ctypes.byref(d)))
+        out = t.empty_like(x)
     if workspace is None:
-        workspace = torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=x.device)
-    _check(load().sdxl_attn_sublayer(ctypes.byref(d), _ptr(x), _ptr(ln_gamma), _ptr(ln_beta), _ptr(w_qkv),
-                                     _ptr(w_qkv_scale), _ptr(w_out), _ptr(b_out), _ptr(out), _ptr(workspace),
-                                     workspace.numel(), _stream(x)))
+        workspace = t.empty((max(sublayer_workspace_bytes(B, S, heads), 1),), dtype=t.uint8, device=x.device)
+    desc = _SUBLAYER_DESC.pack(B, S, heads, E4M3 if w_qkv.dtype == t.uint8 else F16, backend, _f32(eps),
+                               E4M3 if fp8_activations else F16, 0 if ln_fusion else 1)
+    index = x.get_device()
+    _check_packed(load().packed_sdxl_attn_sublayer(
+        desc, x.data_ptr(), _ptr(ln_gamma), _ptr(ln_beta), _ptr(w_qkv), _ptr(w_qkv_scale),
+        _ptr(w_out), _ptr(b_out), out.data_ptr(), workspace.data_ptr(), workspace.numel(),
+        t.raw_stream(index) if index >= 0 else None))
     return out
 
 
@@ -397,7 +440,12 @@ def project_context_kv(context, w_kv, w_kv_scale=None):
     """K | V of the cross-attention context, once per request: context [B, L, C] fp16 against the
     row-concatenated [to_k; to_v] weight [2W, C] (fp16, or uint8 E4M3 with w_kv_scale) -> [B, L, 2W]."""
     B, L, C = context.shape
-    return linear(context.reshape(B * L, C), w_kv, w_scale=w_kv_scale).view(B, L, -1)
+    if not context.is_contiguous():
+        return linear(context.reshape(B * L, C), w_kv, w_scale=w_kv_scale).view(B, L, -1)
+    N = w_kv.shape[0]
+    out = context.new_empty((B, L, N), dtype=(_Torch.loaded or _Torch()).f16)
+    _linear(B * L, C, context, C, w_kv, w_kv_scale, None, None, out, N)
+    return out
 
 
 def cross_attn_sublayer(x, ln_gamma, ln_beta, w_q, w_q_scale, kv, w_out, b_out, heads: int, out=None,
@@ -405,19 +453,22 @@ def cross_attn_sublayer(x, ln_gamma, ln_beta, w_q, w_q_scale, kv, w_out, b_out, 
     """x + to_out(attention(LN(x) . w_q^T, K, V)) for hidden x [B, S, W] fp16 with the context's
     K | V in kv [B, L, 2W] (project_context_kv), the cross-attention half of the reference's
     transformer block (src/cuda/unet.cpp:120-131)."""
-    import torch
+    t = _Torch.loaded or _Torch()
     B, S, W = x.shape
     if out is None:
-        out = torch.empty_like(x)
-    d = CrossSublayerDesc(batch=B, seq=S, heads=heads, ctx_len=kv.shape[1],
-                          w_q_dtype=E4M3 if w_q.dtype == torch.uint8 else F16, attn_backend=backend, ln_eps=eps,
-                          q_activations=E4M3 if fp8_activations else F16)
-    nbytes = int(load().sdxl_cross_attn_sublayer_workspace_bytes(ctypes.byref(d)))
+        out = t.empty_like(x)
+    w_dtype = E4M3 if w_q.dtype == t.uint8 else F16
     if workspace is None:
-        workspace = torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=x.device)
-    _check(load().sdxl_cross_attn_sublayer(ctypes.byref(d), _ptr(x), _ptr(ln_gamma), _ptr(ln_beta), _ptr(w_q),
-                                           _ptr(w_q_scale), _ptr(kv), kv.stride(1), _ptr(w_out), _ptr(b_out),
-                                           _ptr(out), _ptr(workspace), workspace.numel(), _stream(x)))
+        d = CrossSublayerDesc(batch=B, seq=S, heads=heads, ctx_len=kv.shape[1], w_q_dtype=w_dtype)
+        nbytes = int(load().sdxl_cross_attn_sublayer_workspace_bytes(ctypes.byref(d)))
+        workspace = t.empty((max(nbytes, 1),), dtype=t.uint8, device=x.device)
+    desc = _CROSS_SUBLAYER_DESC.pack(B, S, heads, kv.shape[1], w_dtype, backend, _f32(eps),
+                                     E4M3 if fp8_activations else F16)
+    index = x.get_device()
+    _check_packed(load().packed_sdxl_cross_attn_sublayer(
+        desc, x.data_ptr(), _ptr(ln_gamma), _ptr(ln_beta), _ptr(w_q), _ptr(w_q_scale), kv.data_ptr(),
+        kv.stride(1), _ptr(w_out), _ptr(b_out), out.data_ptr(), workspace.data_ptr(), workspace.numel(),
+        t.raw_stream(index) if index >= 0 else None))
     return out
 
 
