@@ -1,12 +1,15 @@
 // K-split projection kernel for fp16 weights (the level-2 output projections
 // of the UNet attention sublayers, 2048 x 1280 x 1280 + bias + residual,
 // src/cuda/unet.cpp:114-118, :128-131, which the reference runs through
-// cuBLASLt, src/cuda/ops_blas.cpp:244-386). Built on its own because its 160 fp32 accumulators per wave stay
+// cuBLASLt, src/cuda/ops_blas.cpp:244-386; and projections of few rows, as the
+// text context's K | V once per request). Built on its own because its 160 fp32 accumulators per wave stay
 // in the accumulation registers: with the MFMA results forced into the
 // architectural VGPRs (the flag the other sublayer kernels build with) the
 // compiler shuffles them between the two register files on every K stage.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <utility>
 
 #include "sublayer_device.hpp"
 #include "sublayer_kernels.hpp"
@@ -19,7 +22,8 @@ typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 
 // K-split projection for fp16 weights: one workgroup = 4 waves = a
 // (32 kMT) x (32 kNT) output tile (64 x 160: the level-2 projections cut
-// into exactly one tile per CU of a 256-CU device). Every
+// into exactly one tile per CU of a 256-CU device; 32 x 32 to 64 x 64: calls of
+// few rows). Every
 // 64-deep K stage of the tile (A rows, then W rows, 128-byte swizzled rows as
 // linear_kernel stages them) is staged once, and wave w takes the 16-deep
 // slice w of every stage for the whole tile: each wave reads each of its
@@ -133,37 +137,33 @@ __global__ __launch_bounds__(256, 1) void linear_ksplit_kernel(LinearParams p) {
                 if (next >= 0) issue(next, q);
         }
     };
+    // stage s landed: at most the transfers of the stages requested after it
+    // (kRing - 2, fewer at the end) still fly
     auto wait_stage = [&](int s) __attribute__((always_inline)) {
         const int later = min(n_stages - 1 - s, kRing - 2);
-        if constexpr (kRing >= 4) {
-            if (later >= 2) wait_vmem<2 * kXfers>();
-            else if (later == 1) wait_vmem<kXfers>();
-            else wait_vmem<0>();
-        } else if constexpr (kRing == 3) {
-            if (later >= 1) wait_vmem<kXfers>();
-            else wait_vmem<0>();
-        } else {
-            wait_vmem<0>();
-        }
+        [&]<int... kLess>(std::integer_sequence<int, kLess...>) __attribute__((always_inline)) {
+            (void)((later >= kRing - 2 - kLess ? (wait_vmem<(kRing - 2 - kLess) * kXfers>(), true) : false) || ...);
+        }(std::make_integer_sequence<int, kRing - 1>{});
     };
 
     // epilogue operands, requested first so that their latency hides under
-    // the loop. Wave w finishes rows 8w .. 8w + 7 of both 32-row m-tiles:
-    // lane l takes row r = 4 (l / 16) + (l / 4) % 4 of those 16 (m-tile r / 8,
-    // row 8w + r % 8) and, in item it (it < kIt), the 8 columns 8 dc .. 8 dc +
-    // 7 with dc = 4 it + l % 4: residual loads and output stores are 16 bytes
-    // per lane, 64 contiguous bytes per row, and the partial reads of every 16
-    // lanes (4 rows x 4 column groups) hit 16 distinct bank groups.
-    static_assert(kMT == 2, "16 rows per wave in the epilogue");
+    // the loop. Wave w finishes rows 8w .. 8w + 7 of the 32-row m-tiles. Two
+    // m-tiles: lane l takes row r = 4 (l / 16) + (l / 4) % 4 of those 16 (m-tile
+    // r / 8, row 8w + r % 8) and, in item it (it < kIt), the 8 columns 8 dc ..
+    // 8 dc + 7 with dc = 4 it + l % 4: residual loads and output stores are 16
+    // bytes per lane, 64 contiguous bytes per row, and the partial reads of
+    // every 16 lanes (4 rows x 4 column groups) hit 16 distinct bank groups.
+    // One m-tile: row l / 8, column groups 8 it + l % 8.
     constexpr int kDC = 4 * kNT;                 // 8-column groups per row
-    constexpr int kIt = kDC / 4;
-    const int er = 4 * (lane >> 4) + ((lane >> 2) & 3);
+    constexpr int kLanes = 8 / kMT;              // lanes per row
+    constexpr int kIt = (kDC + kLanes - 1) / kLanes;
+    const int er = kMT == 2 ? 4 * (lane >> 4) + ((lane >> 2) & 3) : lane >> 3;
     const int ei = er >> 3, erow = 8 * wave + (er & 7);
     f32x4 e_scale[kIt][2];
     f16x8 e_bias[kIt], res[kIt];
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
-        const int dc = 4 * it + (lane & 3);
+        const int dc = kLanes * it + (lane & (kLanes - 1));
         const int en = min(n0 + 8 * dc, p.n - 8);
         const int m = min(m0 + 32 * ei + erow, p.m - 1);
         if (p.w_scale != nullptr) {
@@ -245,21 +245,21 @@ __global__ __launch_bounds__(256, 1) void linear_ksplit_kernel(LinearParams p) {
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
-        const int dc = 4 * it + (lane & 3);
+        const int dc = kLanes * it + (lane & (kLanes - 1));
         const int m = m0 + 32 * ei + erow, en = n0 + 8 * dc;
         const char* part = smem_raw + ei * 4 * kPartBytes + erow * kPartRow;
         const int sw = ((erow >> 1) & 7) ^ (4 * ei);
         f32x4 a[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int off = ((2 * dc + h) ^ sw) << 4;
+            const int off = ((2 * (kDC % kLanes == 0 ? dc : min(dc, kDC - 1)) + h) ^ sw) << 4;
             const f32x4 p0 = *(const lds_f32x4*)(part + off);
             const f32x4 p1 = *(const lds_f32x4*)(part + kPartBytes + off);
             const f32x4 p2 = *(const lds_f32x4*)(part + 2 * kPartBytes + off);
             const f32x4 p3 = *(const lds_f32x4*)(part + 3 * kPartBytes + off);
             a[h] = ((p0 + p1) + p2) + p3;
         }
-        if (m < p.m && en < p.n) {
+        if (m < p.m && en < p.n && (kDC % kLanes == 0 || dc < kDC)) {
             f16x8 o;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -273,36 +273,69 @@ __global__ __launch_bounds__(256, 1) void linear_ksplit_kernel(LinearParams p) {
 
 }  // namespace
 
-bool linear_ksplit_supported(const LinearParams& p, bool w_fp8, int compute_units) {
-    // output projections only (a residual): projections without one (the
-    // query projection) keep linear_kernel's accumulation order, which the
-    // fused query projection + cross-attention reproduces bit for bit
-    if (w_fp8 || p.a_scale != nullptr || p.residual == nullptr || compute_units <= 0 || p.m <= 0 || p.n <= 0)
-        return false;
-    // one round of 64 x 160 tiles that fills at least 90 % of the CUs (the
-    // level-2 projections, 2048 x 1280: 256 tiles); with fewer tiles, or
-    // several per CU, the 64 x 128 kernels measured faster
-    const int64_t tasks = (int64_t)((p.m + 63) / 64) * ((p.n + 159) / 160);
-    if (tasks > compute_units || tasks * 10 < (int64_t)compute_units * 9) return false;
-    auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
-    return p.n % 8 == 0 && p.k % kBK == 0 && p.k > 0 && p.ldc % 8 == 0 && al16(p.c) && p.lda % 8 == 0 &&
-           p.ldw % 8 == 0 && al16(p.a) && al16(p.w) && p.ldr % 8 == 0 && al16(p.residual) &&
-           (p.bias == nullptr || al16(p.bias)) && (p.w_scale == nullptr || al16(p.w_scale)) &&
-           (int64_t)(p.m - 1) * p.lda * 2 + p.k * 2 <= 0xFFFFFFFFll && (int64_t)(p.n - 1) * p.ldw * 2 + p.k * 2 <= 0xFFFFFFFFll;
+namespace {
+
+// Tile of a K-split call, in 32-row and 32-column units.
+struct KsplitTile { int mt, nt; };
+constexpr KsplitTile kNoTile{0, 0};
+
+int64_t tasks_of(const LinearParams& p, KsplitTile t) {
+    return (int64_t)((p.m + 32 * t.mt - 1) / (32 * t.mt)) * ((p.n + 32 * t.nt - 1) / (32 * t.nt));
 }
 
-hipError_t launch_linear_ksplit(const LinearParams& params_in, hipStream_t stream) {
+KsplitTile ksplit_tile(const LinearParams& p, bool w_fp8, int compute_units) {
+    if (w_fp8 || p.a_scale != nullptr || compute_units <= 0 || p.m <= 0 || p.n <= 0) return kNoTile;
+    auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
+    if (!(p.n % 8 == 0 && p.k % kBK == 0 && p.k > 0 && p.ldc % 8 == 0 && al16(p.c) && p.lda % 8 == 0 && p.ldw % 8 == 0 &&
+          al16(p.a) && al16(p.w) && p.ldr % 8 == 0 && al16(p.residual) && al16(p.bias) && al16(p.w_scale) &&
+          (int64_t)(p.m - 1) * p.lda * 2 + p.k * 2 <= 0xFFFFFFFFll && (int64_t)(p.n - 1) * p.ldw * 2 + p.k * 2 <= 0xFFFFFFFFll))
+        return kNoTile;
+    // Few rows (the per-request context K | V, short sequences): the smallest
+    // of the 32 x 32, 32 x 64 and 64 x 64 tiles that fits one round. Their
+    // time is the transfer of a tile's rows over all of K (384 KB at 32 x 64 and
+    // K = 2048, ~53 bytes a cycle), so the more CUs share it the better: [154,
+    // 2048] x [2048, 2560] 60 tiles of 64 x 128 with producer waves 12.0 us,
+    // 200 tiles of 32 x 64 8.8 us; x [1280, 2048] 10.9 -> 7.0 (32 x 32); [200, 640] x
+    // [640, 640] + bias + residual 6.7 -> 4.5; [308, 2048] x [2560, 2048] (64 x 64)
+    // 13.2 -> 13.1.
+    // Projections without a residual only where the attention would run on
+    // 16-row query blocks: beyond, the fused query projection +
+    // cross-attention reproduces linear_kernel's accumulation order bit for bit.
+    if (p.residual != nullptr || short_keys_16_row_blocks((int64_t)((p.m + 31) / 32) * ((p.n + 63) / 64), compute_units))
+        for (KsplitTile t : {KsplitTile{1, 1}, KsplitTile{1, 2}, KsplitTile{2, 2}})
+            if (tasks_of(p, t) <= compute_units) return t;
+    // Output projections (a residual) whose 64 x 160 tiles make one round that
+    // fills at least 90 % of the CUs (the level-2 projections, 2048 x 1280: 256
+    // tiles); with fewer tiles, or several per CU, the 64 x 128 kernels
+    // measured faster.
+    const KsplitTile wide{2, 5};
+    const int64_t tasks = tasks_of(p, wide);
+    return p.residual != nullptr && tasks <= compute_units && tasks * 10 >= (int64_t)compute_units * 9 ? wide : kNoTile;
+}
+
+}  // namespace
+
+bool linear_ksplit_supported(const LinearParams& p, bool w_fp8, int compute_units) {
+    return ksplit_tile(p, w_fp8, compute_units).mt != 0;
+}
+
+hipError_t launch_linear_ksplit(const LinearParams& params_in, int compute_units, hipStream_t stream) {
     LinearParams p = params_in;
-    p.m_blocks = (p.m + 63) / 64;
-    p.n_blocks = (p.n + 159) / 160;
+    const KsplitTile t = ksplit_tile(p, false, compute_units);
+    if (t.mt == 0) return hipErrorInvalidValue;
+    p.m_blocks = (p.m + 32 * t.mt - 1) / (32 * t.mt);
+    p.n_blocks = (p.n + 32 * t.nt - 1) / (32 * t.nt);
     // an XCD's 32 workgroups take 8 m blocks x 4 n blocks (2048 x 1280: 1.3 MB
     // of A rows and 1.6 MB of W rows per XCD's L2)
     p.group_m = p.m_blocks < 8 ? p.m_blocks : 8;
     const dim3 grid((unsigned)((int64_t)p.m_blocks * p.n_blocks)), block(256);
-    if ((int64_t)p.m * p.n * 2 >= kStreamOutBytes)
-        hipLaunchKernelGGL((linear_ksplit_kernel<2, 5, 4, true>), grid, block, 0, stream, p);
-    else
-        hipLaunchKernelGGL((linear_ksplit_kernel<2, 5, 4, false>), grid, block, 0, stream, p);
+    const bool nt = (int64_t)p.m * p.n * 2 >= kStreamOutBytes;
+    // one round: the ring takes what LDS is left
+    if (t.nt == 1) hipLaunchKernelGGL((linear_ksplit_kernel<1, 1, 8, false>), grid, block, 0, stream, p);
+    else if (t.mt == 1) hipLaunchKernelGGL((linear_ksplit_kernel<1, 2, 8, false>), grid, block, 0, stream, p);
+    else if (t.nt == 2) hipLaunchKernelGGL((linear_ksplit_kernel<2, 2, 8, false>), grid, block, 0, stream, p);
+    else if (nt) hipLaunchKernelGGL((linear_ksplit_kernel<2, 5, 4, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((linear_ksplit_kernel<2, 5, 4, false>), grid, block, 0, stream, p);
     return hipGetLastError();
 }
 

@@ -1484,8 +1484,9 @@ hipError_t launch_linear(const LinearParams& params_in, bool w_fp8, int compute_
     // With more tiles per CU (8192 x 640 x 640, 3840 x 1280 x 1280) both
     // measured slower than the plain four-wave kernel.
     // one round of fp16-weight tiles: the K-split kernel (linear_ksplit.hip);
-    // measured 2048 x 1280 x 1280 + bias + residual 15.6 -> 13.8 us
-    if (linear_ksplit_supported(p, w_fp8, compute_units)) return launch_linear_ksplit(p, stream);
+    // measured 2048 x 1280 x 1280 + bias + residual 15.6 -> 13.8 us, context K/V
+    // [154, 2048] x [2048, 2560] 12.0 -> 8.8 us
+    if (linear_ksplit_supported(p, w_fp8, compute_units)) return launch_linear_ksplit(p, compute_units, stream);
     const int cus_lin = compute_units > 0 ? compute_units : 256;
     const bool one_round = tasks <= cus_lin, few = tasks * 4 <= (int64_t)cus_lin * 5;
     if (a_fp8) {

@@ -40,7 +40,7 @@ hipError_t launch_linear(const LinearParams& params, bool w_fp8, int compute_uni
 // and pointers (a, w, c, residual, bias, w_scale) and one round of tiles on
 // compute_units CUs.
 bool linear_ksplit_supported(const LinearParams& params, bool w_fp8, int compute_units);
-hipError_t launch_linear_ksplit(const LinearParams& params, hipStream_t stream);
+hipError_t launch_linear_ksplit(const LinearParams& params, int compute_units, hipStream_t stream);
 // q = a w^T (64 x 128 tiles, one 32-row block of one head per wave), then
 // softmax(q k^T * scale) v per head, written to c. Requires seq % 64 == 0,
 // n % 128 == 0 (heads of 64), 65 <= ctx_len <= 80, k % 64 == 0, no bias or

@@ -225,6 +225,26 @@ def test_linear_k_split(M, N, K, bias):
     assert np.array_equal(host(y), got)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (31, 40, 64), (33, 72, 128), (154, 2560, 2048), (77, 1280, 768),
+                                   (200, 648, 640), (320, 2560, 576), (300, 1000, 1280)])
+@pytest.mark.parametrize("extras", [False, True])
+def test_linear_few_rows(M, N, K, extras):
+    """The 32 x 32, 32 x 64 and 64 x 64 tiles of the K-split kernel: edges of the tile, K below and above its ring."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a = torch.randn(M, K, device=DEV, generator=g).half()
+    w = (torch.randn(N, K, device=DEV, generator=g) / K ** 0.5).half()
+    bias = torch.randn(N, device=DEV, generator=g).half() if extras else None
+    res = torch.randn(M, N, device=DEV, generator=g).half() if extras else None
+    ref = a.double() @ w.double().t()
+    if extras:
+        ref = ref + bias.double() + res.double()
+    out = res.clone() if extras else None  # in place where there is a residual
+    got = sh.linear(a, w, bias=bias, residual=out if extras else None, out=out)
+    # half an fp16 ulp of the result plus fp32 sums of K products of magnitude ~1/sqrt(K)
+    err = (got.double() - ref).abs() - ref.abs() * 2.0 ** -11
+    assert err.max().item() <= 1e-5, err.max().item()
+
+
 def test_linear_k_split_strided():
     """The K-split form on strided operands: a a column slice of a wider buffer, w rows padded, the
     residual and the output column slices of wider buffers (in place and out of place)."""
