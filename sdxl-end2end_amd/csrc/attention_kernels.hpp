@@ -80,7 +80,7 @@ hipError_t launch_online_attention(const OnlineAttentionParams& params, int dtyp
 bool tiled_attention_eligible(const OnlineAttentionParams& params, int dtype);
 hipError_t launch_tiled_attention(const OnlineAttentionParams& params, int dtype, int compute_units, hipStream_t stream);
 
-// FP32 head_dim 512 on the fp32 matrix cores (the VAE mid-block attention):
+// FP32 head_dim 512 on split bf16 planes (the VAE mid-block attention):
 // non-causal, unmasked, 16-byte aligned rows. Same parameters as the online kernel.
 bool attention_f32_d512_eligible(const OnlineAttentionParams& params, int dtype);
 hipError_t launch_attention_f32_d512(const OnlineAttentionParams& params, int compute_units, hipStream_t stream);

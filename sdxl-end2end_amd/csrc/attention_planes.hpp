@@ -55,12 +55,5 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t (&out)[kN]) {
     }
 }
 
-// NaN if the packed pair holds an infinity or a NaN, else x unchanged.
-template <bool kF16>
-__device__ __forceinline__ float probe(uint32_t pair, float x) {
-    if constexpr (kF16) return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pair), f16x2{0, 0}, x, false);
-    else return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), bf16x2{0, 0}, x, false);
-}
-
 }  // namespace
 }  // namespace sdxl_hip

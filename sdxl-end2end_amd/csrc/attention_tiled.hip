@@ -22,25 +22,27 @@
 // the score registers). The key groups of a query block merge through LDS.
 //
 // Measured (graph replay): FP32 [1, 20, 1024, 64] 1943 us on the per-row kernel,
-// 64 us here (84 TFLOP/s; the fp32 matrix cores' peak is 157); FP32
-// [2, 8, 1000, 160] 98 us, fp16 [2, 8, 1000, 80] 1676 -> 29.5 us. Against 64 bits
-// the FP32 result is closer than the per-row kernel's (2.8e-7 against 6.5e-7 of
+// 58 us here (92 TFLOP/s; the fp32 matrix cores' peak is 157); FP32
+// [2, 8, 1000, 160] 91 us, fp16 [2, 8, 1000, 80] 1676 -> 28.5 us. Against 64 bits
+// the FP32 result is closer than the per-row kernel's (4.1e-7 against 6.4e-7 of
 // the output's norm at 1024 keys). Per wave and sub-tile 48 MFMAs (1536 cycles)
-// meet ~450 other vector instructions (~1800 cycles: the split of the stage's
+// meet ~400 other vector instructions (~1600 cycles: the split of the stage's
 // share and of the probabilities, the softmax); two waves per SIMD overlap
-// them in part.
+// them in part. Looking for special values in the results instead of while
+// splitting took 4-17 % off every shape (61.3 -> 58.3, 20.8 -> 17.3 us at
+// [4, 20, 1024 x 77, 80]).
 //
 // LDS rows are 64-dim panels of 128 bytes, 16-byte chunks XOR-swizzled by row.
 //
 // Values that planes cannot carry (infinities, NaN, fp32 above the largest
-// bf16) are found while splitting; their workgroup then runs its remaining
-// stages on plain fp32 arithmetic from global memory (slow, the same results
-// as the per-row kernel).
+// bf16) leave NaN in the results; a query block with any runs the per-row
+// kernel's code instead (attention_row.hpp).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "attention_kernels.hpp"
 #include "attention_planes.hpp"
+#include "attention_row.hpp"
 
 namespace sdxl_hip {
 namespace {
@@ -96,22 +98,19 @@ __device__ __forceinline__ Raw<T> load8(const char* base, uint32_t off, int d0, 
     return r;
 }
 
-// Planes of eight loaded values (out[plane]) and, in bad, NaN if any of them
-// cannot be carried by planes.
+// Planes of eight loaded values (out[plane]).
 template <typename T>
-__device__ __forceinline__ void planes8(const Raw<T>& r, u32x4 (&out)[Planes<T>::in], float& bad) {
+__device__ __forceinline__ void planes8(const Raw<T>& r, u32x4 (&out)[Planes<T>::in]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if constexpr (sizeof(T) == 4) {
             uint32_t w[3];
             split2<3, false>(__builtin_bit_cast(float, (uint32_t)r.v[i >> 1][2 * (i & 1)]),
                              __builtin_bit_cast(float, (uint32_t)r.v[i >> 1][2 * (i & 1) + 1]), w);
-            bad = probe<false>(w[1], bad);
 #pragma unroll
             for (int pl = 0; pl < 3; ++pl) out[pl][i] = w[pl];
         } else {
             out[0][i] = r.v[0][i];
-            bad = probe<Planes<T>::f16>(r.v[0][i], bad);
         }
     }
 }
@@ -124,6 +123,13 @@ __device__ __forceinline__ void zero_past(u32x4 (&pl)[kN], int n) {
     for (int i = 0; i < kN; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) pl[i][e] = 2 * e >= n ? 0u : 2 * e + 1 >= n ? pl[i][e] & 0xFFFFu : pl[i][e];
+}
+
+// A row in plain fp32 (out of line: it leaves the tiled kernel's registers alone).
+template <typename T>
+__device__ __attribute__((noinline)) void plain_row(const T* q, const T* k, const T* v, T* o, int64_t k_stride, int64_t v_stride,
+                                                    const int32_t* mask, int n_keys, int dim, float scale, float* qs) {
+    row_attention<T, 3>(q, k, v, o, k_stride, v_stride, mask, n_keys, dim, scale, qs);
 }
 
 constexpr int tiled_panels(int dp) { return (dp + 63) / 64; }
@@ -149,7 +155,6 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
     constexpr int kLdsBytes = 2 * kKS * kSub > kMergeBytes ? 2 * kKS * kSub : kMergeBytes;
     static_assert(kLdsBytes <= 160 * 1024 - 64, "LDS");
     __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];
-    __shared__ int special;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -172,9 +177,6 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
     const T* vbase = (const T*)p.v + (int64_t)b * p.k_seq * p.v_row_stride + (int64_t)h * D;
     T* obase = (T*)p.o + (int64_t)b * p.q_seq * p.o_row_stride + (int64_t)h * D;
 
-    if (threadIdx.x == 0) special = 0;
-    __syncthreads();
-
     int n_keys = p.k_seq;
     if (p.causal) n_keys = min(n_keys, wg_q0 + 32 * kQB);
     const int n_stages = (n_keys + kKS * kKeys - 1) / (kKS * kKeys);
@@ -183,7 +185,6 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
     const int my_query = q0 + col;
     i16x8 qop[kIn][kSteps];
     {
-        float bad = 0.0f;
         const uint32_t off = (uint32_t)min(my_query - wg_q0, p.q_seq - 1 - wg_q0) * (uint32_t)(p.q_row_stride * (int64_t)sizeof(T));
         const char* src = (const char*)(qbase + (int64_t)wg_q0 * p.q_row_stride);
 #pragma unroll
@@ -191,12 +192,11 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
             const int d0 = 16 * ks + 8 * hf;
             const Raw<T> r = load8<T, kVec>(src, off, d0, D);
             u32x4 pl[kIn];
-            planes8<T>(r, pl, bad);
+            planes8<T>(r, pl);
             zero_past<kIn>(pl, D - d0);
 #pragma unroll
             for (int i = 0; i < kIn; ++i) qop[i][ks] = __builtin_bit_cast(i16x8, pl[i]);
         }
-        if (kIn > 1 && bad != bad) atomicOr(&special, 1);
     }
 
     // Stage loads: chunk n of the stage is row n / kChunks (sub-tile row / 32),
@@ -218,7 +218,6 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
             mask_word = p.key_mask[(int64_t)b * p.k_seq + min(key0 + kKeys * kg + col, p.k_seq - 1)];
     };
     auto write_stage = [&]() __attribute__((always_inline)) {
-        float bad_k = 0.0f, bad_v = 0.0f;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const int n = threadIdx.x + 256 * i;
@@ -227,19 +226,17 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
                 const int row = srow % kKeys;
                 char* dst = lds + (srow / kKeys) * (2 * kSub) + (chunk >> 3) * kPanelBytes + row * 128 + (((chunk & 7) ^ swz(row)) << 4);
                 u32x4 pl[kIn];
-                planes8<T>(kraw[i], pl, bad_k);
+                planes8<T>(kraw[i], pl);
                 // K past D: what load8 put there is the row's own, but an
-                // infinity among it would meet Q's zeros (FP32: found above)
+                // infinity among it would meet Q's zeros (FP32: planes make it NaN)
                 if (kIn == 1 && D != kDp) zero_past<kIn>(pl, D - 8 * chunk);
 #pragma unroll
                 for (int j = 0; j < kIn; ++j) *(lds_u32x4*)(dst + j * kPlane) = pl[j];
-                planes8<T>(vraw[i], pl, bad_v);
+                planes8<T>(vraw[i], pl);
 #pragma unroll
                 for (int j = 0; j < kIn; ++j) *(lds_u32x4*)(dst + kSub + j * kPlane) = pl[j];
             }
         }
-        if (kIn > 1 && bad_k != bad_k) atomicOr(&special, 1);
-        if (bad_v != bad_v) atomicOr(&special, 2);
     };
 
     // Operand offsets in a panel: K row col, chunk (2 (ks & 3) + hf) ^ swz(col);
@@ -279,38 +276,22 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
         write_stage();
         __syncthreads();
         if (s + 1 < n_stages) load_stage(s + 1);
-        const int slow = __builtin_amdgcn_readfirstlane(special);
         // nothing visible to any of the wave's queries
         if (vis == 0u || (p.causal && key0 > q0 + 31)) continue;
 
         f32x16 sc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
-        if (__builtin_expect(slow & 1, 0)) {
-            // keys one at a time (uniform loop): nothing of it stays in registers
-            const T* qrow = qbase + (int64_t)min(my_query, p.q_seq - 1) * p.q_row_stride;
-#pragma unroll 1
-            for (int i = 0; i < 16; ++i) {
-                const int key = min(key0 + 8 * (i >> 2) + 4 * hf + (i & 3), p.k_seq - 1);
-                const T* krow = kbase + (int64_t)key * p.k_row_stride;
-                float dot = 0.0f;
-#pragma unroll 1
-                for (int d = 0; d < D; ++d) dot += (float)qrow[d] * (float)krow[d];
 #pragma unroll
-                for (int e = 0; e < 16; ++e) sc[e] = e == i ? dot : sc[e];
-            }
-        } else {
+        for (int ks = 0; ks < kSteps; ++ks) {
+            const char* src = ksub + (ks >> 2) * kPanelBytes + col * 128 + (((2 * (ks & 3) + hf) ^ k_swz) << 4);
+            i16x8 kop[kIn];
 #pragma unroll
-            for (int ks = 0; ks < kSteps; ++ks) {
-                const char* src = ksub + (ks >> 2) * kPanelBytes + col * 128 + (((2 * (ks & 3) + hf) ^ k_swz) << 4);
-                i16x8 kop[kIn];
+            for (int i = 0; i < kIn; ++i) kop[i] = *(const lds_i16x8*)(src + i * kPlane);
 #pragma unroll
-                for (int i = 0; i < kIn; ++i) kop[i] = *(const lds_i16x8*)(src + i * kPlane);
+            for (int i = kIn - 1; i >= 0; --i)
 #pragma unroll
-                for (int i = kIn - 1; i >= 0; --i)
-#pragma unroll
-                    for (int j = kIn - 1 - i; j >= 0; --j) sc = mfma32<kF16>(kop[i], qop[j][ks], sc);
-            }
+                for (int j = kIn - 1 - i; j >= 0; --j) sc = mfma32<kF16>(kop[i], qop[j][ks], sc);
         }
 
         if (vis != ~0u || (p.causal && key0 + 31 > q0)) {
@@ -349,37 +330,14 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
                 float x = sc[i] * c;
                 asm("" : "+v"(x));  // rounded: no fused multiply-add
                 x -= m_run;
+                // a NaN that came with no finite score must still reach the check below
+                if (m_run == -__builtin_inff() && sc[i] != sc[i]) l_run = sc[i];
                 pr[i] = m_run == -__builtin_inff() ? 0.0f : fabsf(m_run) <= 1.0e6f ? pr[i] : __builtin_amdgcn_exp2f(x + Planes<T>::shift);
             }
         }
 #pragma unroll
         for (int i = 0; i < 16; i += 4) l_run += (pr[i] + pr[i + 1]) + (pr[i + 2] + pr[i + 3]);
 
-        if (__builtin_expect(slow & 2, 0)) {
-            // plain products from global memory, keys in the lanes' order
-#pragma unroll 1
-            for (int n = 0; n < 32; ++n) {
-                const int i = n >> 1, half = n & 1;
-                const int key = key0 + 8 * (i >> 2) + 4 * half + (i & 3);
-                float pj = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 16; ++e) pj = e == i ? pr[e] : pj;
-                pj = __shfl(pj, col + 32 * half, 64);
-                if (key >= n_keys) continue;
-                const T* vrow = vbase + (int64_t)key * p.v_row_stride;
-#pragma unroll
-                for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        int d = 4 * hf;  // opaque, one at a time: no registers held for this path
-                        asm volatile("" : "+v"(d));
-                        d = min(d + 32 * t + 8 * (e >> 2) + (e & 3), D - 1);
-                        acc[t][e] += pj * (float)vrow[d];
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-            }
-            continue;
-        }
 #pragma unroll
         for (int ss = 0; ss < 2; ++ss) {
             i16x8 pop[kProb];
@@ -441,6 +399,26 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
     }
 
     const float inv = 1.0f / fmaxf(l_tot, 1.0e-20f);
+    // Planes turn an infinity, a NaN or an FP32 value above the largest bf16
+    // into a NaN, which reaches every score or output that it meets: a query
+    // block with one (or whose results overflow) starts over in plain fp32.
+    float bad = l_tot;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            acc[t][i] *= inv;
+            bad = __builtin_fmaf(acc[t][i], 0.0f, bad);
+        }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad != bad) != 0, 0)) {
+        __shared__ float row_q[4][kDp];
+#pragma unroll 1
+        for (int r = 0; r < 32 && q0 + r < p.q_seq; ++r)
+            plain_row<T>(qbase + (int64_t)(q0 + r) * p.q_row_stride, kbase, vbase, obase + (int64_t)(q0 + r) * p.o_row_stride,
+                         p.k_row_stride, p.v_row_stride, p.key_mask != nullptr ? p.key_mask + (int64_t)b * p.k_seq : nullptr,
+                         p.causal ? min(p.k_seq, q0 + r + 1) : p.k_seq, D, p.scale, row_q[wave]);
+        return;
+    }
     if (my_query >= p.q_seq) return;
     T* orow = obase + (int64_t)my_query * p.o_row_stride;
 #pragma unroll
@@ -450,7 +428,7 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
             const int d0 = 32 * t + 8 * u + 4 * hf;
             T w[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = (T)(acc[t][4 * u + e] * inv);
+            for (int e = 0; e < 4; ++e) w[e] = (T)acc[t][4 * u + e];
             if constexpr (kVec) {
                 if (d0 < D) {
                     if constexpr (sizeof(T) == 4) *(f32x4*)(orow + d0) = f32x4{(float)w[0], (float)w[1], (float)w[2], (float)w[3]};
@@ -475,7 +453,7 @@ hipError_t launch_one(const OnlineAttentionParams& p, hipStream_t stream) {
 }
 
 // Key groups per workgroup. Two (64 queries share a stage's split) is the
-// general choice: the FP32 [1, 20, 1024, 64] call takes 64 us with two, 73 with
+// general choice: the FP32 [1, 20, 1024, 64] call took 64 us with two, 73 with
 // one; fp16 [2, 8, 1000, 80] 29.5 with two, 47 with one. One (128 queries) for
 // short key sequences on full grids, where a wave has few sub-tiles to merge
 // (fp16 [4, 20, 1024 x 77, 80] 19.5 against 21.9 us). Four (32 queries) for

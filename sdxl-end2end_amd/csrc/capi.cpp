@@ -218,7 +218,7 @@ sdxl_status sdxl_attn_fwd(const sdxl_attn_desc* d, const void* q, const void* k,
         p.batch = (int32_t)d->batch; p.q_seq = (int32_t)d->q_seq; p.k_seq = (int32_t)d->k_seq;
         p.heads = (int32_t)d->heads; p.head_dim = (int32_t)d->head_dim; p.causal = d->causal != 0;
         p.scale = scale;
-        // FP32 at head_dim 512 (the VAE's attention) runs on the fp32 matrix
+        // FP32 at head_dim 512 (the VAE's attention) runs on the bf16 matrix
         // cores when the call allows (auto backend, no mask, non-causal,
         // aligned rows), head_dim <= 160 on the tiled kernel; an explicit
         // warp-online request keeps the per-row kernel.
