@@ -139,8 +139,8 @@ constexpr int tiled_lds(int dp, int ks) { return 2 * ks * Planes<T>::in * tiled_
 template <typename T>
 constexpr int tiled_occupancy(int dp) { return sizeof(T) == 4 ? (dp <= 64 ? 2 : 1) : (dp <= 64 ? 3 : dp <= 128 ? 2 : 1); }
 
-template <typename T, int kDp, int kKS, bool kVec>
-__global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_kernel(OnlineAttentionParams p, int q_blocks) {
+template <typename T, int kDp, int kKS, bool kVec, int kOcc>
+__global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttentionParams p, int q_blocks) {
     constexpr int kIn = Planes<T>::in, kProb = Planes<T>::prob;
     constexpr bool kF16 = Planes<T>::f16;
     constexpr int kPanels = tiled_panels(kDp);
@@ -442,13 +442,13 @@ __global__ __launch_bounds__(256, tiled_occupancy<T>(kDp)) void tiled_attention_
         }
 }
 
-template <typename T, int kDp, int kKS, bool kVec>
+template <typename T, int kDp, int kKS, bool kVec, int kOcc = tiled_occupancy<T>(kDp)>
 hipError_t launch_one(const OnlineAttentionParams& p, hipStream_t stream) {
     constexpr int kRows = 128 / kKS;
     const int64_t q_blocks = ((int64_t)p.q_seq + kRows - 1) / kRows;
     const int64_t grid = q_blocks * p.heads * p.batch;
     if (grid > INT32_MAX) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((tiled_attention_kernel<T, kDp, kKS, kVec>), dim3((unsigned)grid), dim3(256), 0, stream, p, (int)q_blocks);
+    hipLaunchKernelGGL((tiled_attention_kernel<T, kDp, kKS, kVec, kOcc>), dim3((unsigned)grid), dim3(256), 0, stream, p, (int)q_blocks);
     return hipGetLastError();
 }
 
@@ -470,6 +470,14 @@ hipError_t launch_dp(const OnlineAttentionParams& p, int compute_units, bool vec
         if (p.k_seq > 2 * kKeys && blocks < 2 * cus) return launch_one<T, kDp, 4, true>(p, stream);
     }
     if (p.k_seq <= kKeys || (p.k_seq <= 4 * kKeys && blocks >= 8 * cus)) return launch_one<T, kDp, 1, true>(p, stream);
+    // FP32 with more than two workgroups per CU: three waves per SIMD in place
+    // of two, although their registers spill ([1, 10, 4096, 64] 330 -> 294 us,
+    // [2, 20, 1024, 64] 89.7 -> 81.8, [2, 20, 900, 48] 83 -> 74); with two at
+    // most it loses ([2, 16, 1000, 64], exactly two, 58.6 -> 63.1).
+    if constexpr (sizeof(T) == 4 && kDp == 64) {
+        const int64_t workgroups = ((int64_t)p.q_seq + 63) / 64 * p.heads * p.batch;
+        if (workgroups > 2 * cus) return launch_one<T, kDp, 2, true, 3>(p, stream);
+    }
     return launch_one<T, kDp, 2, true>(p, stream);
 }
 

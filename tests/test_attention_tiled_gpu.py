@@ -51,7 +51,7 @@ def check(got, ref, dtype):
     (1, 3, 64, 127, 64), (2, 2, 63, 128, 72), (1, 2, 130, 129, 96), (1, 2, 33, 200, 128),
     (1, 2, 70, 31, 136), (2, 1, 97, 300, 160),
     (1, 3, 50, 77, 7), (1, 2, 66, 90, 33), (2, 2, 40, 70, 50), (1, 2, 35, 100, 159),  # rows not 16-byte aligned
-    (2, 40, 1000, 70, 40), (1, 20, 900, 260, 64)])  # one and two key groups on full grids
+    (2, 40, 1000, 70, 40), (1, 20, 900, 260, 64), (1, 33, 1000, 150, 56)])  # one and two key groups on full grids
 def test_tiled_shapes(B, H, Sq, Sk, D, dtype):
     if dtype != "f32" and D == 64:
         D = 56  # 16-bit head_dim 64 runs elsewhere
