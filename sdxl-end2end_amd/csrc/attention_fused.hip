@@ -344,7 +344,9 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     // last stage can lack keys of either half.
     const int key_groups = split2 ? (n_keys + kKeyTile - 1) / kKeyTile : (n_keys + 31) / 32;
     const int half_keys = (split2 ? kKeyTile : 32) * (key_groups >> 1);
-    const int n_tiles = split ? (key_groups + 1) >> 1 : (n_keys + kKeyTile - 1) / kKeyTile;
+    const int n_tiles = split              ? (key_groups + 1) >> 1
+                        : mixed && !kTail ? p.k_seq / kKeyTile
+                                          : (n_keys + kKeyTile - 1) / kKeyTile;
     const int key_end = split && khalf == 0 ? half_keys : n_keys;  // of this wave's part
     // ---- tile transfers: the 16 1-KiB transfers of a K tile plus a V tile are
     // split over the waves; transfer n covers the 8-row slab n%8 (rows
@@ -518,7 +520,12 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     const int slab = (i & 1) + 4 * (i >> 1) + 2 * j;
-                    mixed_slab(set_v1, vs_bytes, vt, slab, buf);
+                    if constexpr (kTail) {
+                        mixed_slab(set_v1, vs_bytes, vt, slab, buf);
+                    } else {
+                        const char* slab_base = set_v1 + (int64_t)(vt * kKeyTile + 8 * slab) * vs_bytes;
+                        lds_dma16(slab_base, mixed_off, lds_addr(buf + 8 * slab * kRowBytes));
+                    }
                 }
             }
         }
