@@ -170,11 +170,17 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     if (threadIdx.x == 0) special = 0;
     __syncthreads();
 
-    // Buffer descriptor of the wave's slice of the rows of block t; rows past
-    // k_seq read zeros (K: their scores are hidden; V: zero probabilities).
+    // Block t is rows first_row(t) .. +31: a last block that k_seq does not fill
+    // starts earlier, at k_seq - 32, and hides the keys that the block before it
+    // had, so that every load is of a row that exists (the range check of a
+    // load subtracts its scalar offset without a borrow and cannot be relied
+    // on). Fewer than 32 keys in all: K rows past the end are caught by that
+    // check (their offset is per lane and the scalar one below the size), V by
+    // load_v_short.
+    auto first_row = [&](int t) __attribute__((always_inline)) { return max(min(t * kKeys, p.k_seq - kKeys), 0); };
     auto block_rows = [&](const char* slice, uint32_t stride_b, int t, int dims) __attribute__((always_inline)) {
-        const int rows = min(kKeys, p.k_seq - t * kKeys);
-        return __builtin_amdgcn_make_buffer_rsrc((void*)(slice + (int64_t)t * kKeys * stride_b), 0,
+        const int rows = min(kKeys, p.k_seq);
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(slice + (int64_t)first_row(t) * stride_b), 0,
                                                  (int)((uint32_t)(rows - 1) * stride_b + 4u * dims), 0x00027000);
     };
     // K of block t, K steps 2 half and 2 half + 1: lane holds key col, dims
@@ -205,6 +211,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
                 vraw[ss][e][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, v_off, (16 * ss + e) * v_stride_b, 0));
             }
         }
+    };
+    auto load_v_short = [&](int ss) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int dt = 0; dt < kDT; ++dt)
+                vraw[ss][e][dt] = *(const float*)(vslice + ((uint32_t)min(16 * ss + 8 * hf + e, p.k_seq - 1) * v_stride_b + 4u * (kDT * col + dt)));
     };
     load_k(0, 0);
     load_k(0, 1);
@@ -368,10 +381,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
             sc[i] = half == 0 ? x : sc[i] + x;
         }
     };
-    auto softmax = [&](int t) __attribute__((always_inline)) {
-        const int lim = p.k_seq - t * kKeys - (8 * su + 4 * sh + sr);
+    auto softmax = [&]<bool kLast>(int t) __attribute__((always_inline)) {
+        if constexpr (kLast) {
+            // visible: keys of the last block from t kKeys on, below k_seq
+            const int before = t * kKeys - first_row(t), n = min(p.k_seq, kKeys);
+            const int mine = 8 * su + 4 * sh + sr;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) sc[i] = i < lim ? sc[i] : -__builtin_inff();
+            for (int i = 0; i < kPer; ++i) sc[i] = mine + i >= before && mine + i < n ? sc[i] : -__builtin_inff();
+        }
         float mx = sc[0];
 #pragma unroll
         for (int i = 1; i < kPer; ++i) mx = fmaxf(mx, sc[i]);
@@ -408,8 +425,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     read_qlow(0);
     Operand even = {}, odd = {};
     if constexpr (kQT == 1) {
-        load_v(0, 0);
-        load_v(0, 1);
+        if (p.k_seq < kKeys) {
+            load_v_short(0);
+            load_v_short(1);
+        } else {
+            load_v(0, 0);
+            load_v(0, 1);
+        }
     }
     if (n_blocks > 1) {
         load_k(1, 0);
@@ -462,7 +484,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
         sum_partials(1);
         scores_stage.template operator()<2>(even, [&]() __attribute__((always_inline)) {
             odd = split_k(3);
-            softmax(t);
+            softmax.template operator()<false>(t);
         });
         if constexpr (kQT == 2) load_v(t, 1);
         else load_k(t2, 1);
@@ -502,7 +524,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     sum_partials(0);
     read_partials(1);
     sum_partials(1);
-    softmax(n_blocks - 1);
+    softmax.template operator()<true>(n_blocks - 1);
     __syncthreads();
     rescale();
 #pragma unroll
@@ -582,10 +604,11 @@ hipError_t launch_attention_f32_d512(const OnlineAttentionParams& p, int compute
     const int64_t cus = compute_units > 0 ? compute_units : 256;
     const int64_t b64 = ((int64_t)p.q_seq + 63) / 64, b32 = ((int64_t)p.q_seq + 31) / 32;
     const int64_t r64 = (b64 * heads_total + cus - 1) / cus, r32 = (b32 * heads_total + cus - 1) / cus;
-    const int64_t grid = (5 * r64 <= 3 * r32 ? b64 : 2 * b32 * heads_total <= cus ? 2 * b32 : b32) * heads_total;
+    const bool wide = 5 * r64 <= 3 * r32 && p.k_seq >= kKeys;  // 64 queries: no short last block
+    const int64_t grid = (wide ? b64 : 2 * b32 * heads_total <= cus ? 2 * b32 : b32) * heads_total;
     if (grid > INT32_MAX) return hipErrorInvalidValue;
     const dim3 g((unsigned)grid), block(kWaves * 64);
-    if (5 * r64 <= 3 * r32) hipLaunchKernelGGL((attention_f32_d512_kernel<2, 2>), g, block, 0, stream, p, (int)b64);
+    if (wide) hipLaunchKernelGGL((attention_f32_d512_kernel<2, 2>), g, block, 0, stream, p, (int)b64);
     else if (2 * b32 * heads_total <= cus) hipLaunchKernelGGL((attention_f32_d512_kernel<1, 1>), g, block, 0, stream, p, (int)b32);
     else hipLaunchKernelGGL((attention_f32_d512_kernel<1, 2>), g, block, 0, stream, p, (int)b32);
     return hipGetLastError();
