@@ -33,12 +33,12 @@
 // worked while the other did (3.33 against 2.73 ms at 16384 tokens).
 //
 // Bound: at 64 queries the bf16 matrix cores, busy 72 % of a block's ~8500
-// cycles at a power-limited ~1.7 GHz (1.29 PFLOP/s of plane products; the
+// cycles at a power-limited ~1.7 GHz (1.25 PFLOP/s of plane products; the
 // vendor's bf16 GEMM reaches 1.16 on the same card); at 32 the split's vector
 // instructions and the exchange of the partials (MFMA 3072 of ~6800 cycles).
 // Measured against fp32 matrix instructions (v_mfma_f32_32x32x2, the same
 // outputs within 64-bit error 2.0e-6 here, 2.3e-6 there): 16384 tokens 5.02 ->
-// 2.56 ms (215 TFLOP/s), 8192 1.43 -> 0.89, 4096 0.403 -> 0.349 (two
+// 2.64 ms (208 TFLOP/s), 8192 1.43 -> 0.90, 4096 0.403 -> 0.353 (two
 // workgroups per block; one: 0.400), 1024 105 -> 83 us. Tried and not kept:
 // the residuals x - h by v_dot2 (fewer instructions, but wait states: 2.92
 // ms), K loads of 64-byte row segments exchanged by v_permlane16_swap (4096
@@ -141,7 +141,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     constexpr int kPer = 2 * kQT;                // scores per lane of the summed block
     constexpr int kGroup = kKeys / kPer;         // lanes per query there
     constexpr int kPartBytes = kWaves * kQT * 4 * 1024;
-    constexpr int kQlBytes = kQT == 2 ? kWaves * kQT * kSteps * 1024 : 0;
+    // kQT = 2: the third plane of every K step and the second of the last one
+    // (registers that would spill) wait in LDS
+    constexpr int kQlBytes = kQT == 2 ? kWaves * kQT * (kSteps + 1) * 1024 : 0;
     constexpr int kProbBytes = kQT * 2 * 3 * 1024;
     __shared__ __attribute__((aligned(16))) char part[kPartBytes];  // [wave][tile][4][64] x 16 bytes
     __shared__ __attribute__((aligned(16))) char qlow[kQlBytes + 16];
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
 
     // Q planes: lane holds query q0 + 32 qt + col, dims 16 ks + 8 hf .. +7.
     i16x8 qop[kQT][kSteps][kRegPlanes];
-    char* const qlow_mine = qlow + (kQT == 2 ? wave * kQT * kSteps * 1024 : 0) + lane * 16;
+    char* const qlow_mine = qlow + (kQT == 2 ? wave * kQT * (kSteps + 1) * 1024 : 0) + lane * 16;
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt) {
         const float* row = qhead + (int64_t)min(q0 + 32 * qt + col, p.q_seq - 1) * p.q_row_stride + kSlice * wave + 8 * hf;
@@ -241,7 +243,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
             }
 #pragma unroll
             for (int j = 0; j < kRegPlanes; ++j) qop[qt][ks][j] = __builtin_bit_cast(i16x8, pl[j]);
-            if constexpr (kQT == 2) *(lds_u32x4*)(qlow_mine + (qt * kSteps + ks) * 1024) = pl[2];
+            if constexpr (kQT == 2) {
+                *(lds_u32x4*)(qlow_mine + (qt * (kSteps + 1) + ks) * 1024) = pl[2];
+                if (ks == kSteps - 1) *(lds_u32x4*)(qlow_mine + (qt * (kSteps + 1) + kSteps) * 1024) = pl[1];
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -286,7 +291,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     auto read_qlow = [&](int ks) __attribute__((always_inline)) {
         if constexpr (kQT == 2)
 #pragma unroll
-            for (int qt = 0; qt < kQT; ++qt) qlo[qt] = __builtin_bit_cast(i16x8, *(const lds_u32x4*)(qlow_mine + (qt * kSteps + ks) * 1024));
+            for (int qt = 0; qt < kQT; ++qt) qlo[qt] = __builtin_bit_cast(i16x8, *(const lds_u32x4*)(qlow_mine + (qt * (kSteps + 1) + ks) * 1024));
     };
     auto scores_step = [&](int ks, const Operand& k, const i16x8 (&low)[kQT]) __attribute__((always_inline)) {
 #pragma unroll
@@ -294,11 +299,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
             i16x8 ql;
             if constexpr (kQT == 2) ql = low[qt];
             else ql = qop[qt][ks][2];
+            i16x8 qm = qop[qt][ks][1];
+            if constexpr (kQT == 2)
+                if (ks == kSteps - 1) qm = __builtin_bit_cast(i16x8, *(const lds_u32x4*)(qlow_mine + (qt * (kSteps + 1) + kSteps) * 1024));
             s[qt] = mfma32<false>(k.pl[2], qop[qt][ks][0], s[qt]);
-            s[qt] = mfma32<false>(k.pl[1], qop[qt][ks][1], s[qt]);
+            s[qt] = mfma32<false>(k.pl[1], qm, s[qt]);
             s[qt] = mfma32<false>(k.pl[1], qop[qt][ks][0], s[qt]);
             s[qt] = mfma32<false>(k.pl[0], ql, s[qt]);
-            s[qt] = mfma32<false>(k.pl[0], qop[qt][ks][1], s[qt]);
+            s[qt] = mfma32<false>(k.pl[0], qm, s[qt]);
             s[qt] = mfma32<false>(k.pl[0], qop[qt][ks][0], s[qt]);
         }
     };
