@@ -626,12 +626,15 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     // otherwise stall the wave on the chain). At the end, the K operands of
     // the group after next (tile buffer kn2, group g2) are prefetched into kop.
     // Modes: kPlain: each half is checked for overflow after the fact; kFirst:
-    // exact maximum over the whole group first (a row's first group); kHide: as
-    // kPlain, unless hide (wave-uniform) is set: then keys outside the
-    // visibility word or the causal limit are hidden and the maximum is exact
-    // (a branch to code out of line, as the anchor update: the steps of ragged
-    // and masked calls keep the plain step's registers); kLast: hide without the
-    // branch.
+    // exact maximum over the whole group first (a row's first group); kHide: if
+    // hide (wave-uniform) is set, keys outside the visibility word or the causal
+    // limit are hidden and the maximum is exact (a branch to code out of line,
+    // as the anchor update: the steps of ragged calls keep the plain step's
+    // registers), else as kPlain, or, in masked calls, as kFirst: there the
+    // running maximum stays exact, so that a row's largest weight is 1 and
+    // carries no rounding ([2, 16, 1500], distance from 64 bits: key mask 2.76e-4
+    // exact, 2.89e-4 against a stale anchor; causal 2.49e-4, 2.54e-4); kLast:
+    // hide without the branch.
     auto group_step = [&]<int kMode, bool kPrefetchK = true>(f32x16& s_cur, f32x16& s_next, i16x8 (&kop)[4], const char* vb,
                                                      int g, bool hide, int key0, uint64_t vis, const char* kn2, int g2) __attribute__((always_inline)) {
         // V^T operands of both 16-key halves in their own registers; the second
@@ -639,6 +642,7 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
         // before them, c3 94.1 -> 93.8 us, c1 17.1 -> 16.9 us)
         i16x8 vop[2], vop1[2];
         load_v(vb, g, 0, vop);
+        constexpr bool kExact = kMode == kFirst || kMode == kLast || (kMaskAll && kMode == kHide);
         if constexpr (kMode == kHide || kMode == kLast) {
             if (kMode == kLast || __builtin_expect(hide, 0)) {
                 const uint32_t lane_vis = (uint32_t)(vis >> (32 * g + 4 * hf));
@@ -650,18 +654,21 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
                     const bool ok = ((lane_vis >> kk) & 1u) && (kk <= causal_lim);
                     s_cur[i] = ok ? s_cur[i] : -__builtin_inff();
                 }
-                const float shift = exact_max(s_cur, 0, 16);
+                if constexpr (!kExact) {
+                    const float shift = exact_max(s_cur, 0, 16);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) s_cur[i] -= shift;
+                    for (int i = 0; i < 16; ++i) s_cur[i] -= shift;
+                }
             }
-        } else if constexpr (kMode == kFirst) {
+        }
+        if constexpr (kExact) {
             const float shift = exact_max(s_cur, 0, 16);
 #pragma unroll
             for (int i = 0; i < 16; ++i) s_cur[i] -= shift;
         }
         float e[16];
         uint32_t pk[8];
-        constexpr bool kCheck = kMode != kFirst && kMode != kLast;
+        constexpr bool kCheck = !kExact;
 
         // Eight slots, each one MFMA followed by about its duration (32 cycles)
         // of VALU work that does not depend on it, pinned with scheduling
@@ -1072,11 +1079,12 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
 }
 
 // Ragged and masked calls (kTail, kMaskAll) decide per group, by a wave-uniform
-// branch, whether keys have to be hidden, so that their other groups take the
-// plain step: masked causal fp16 [2, 16, 1500] 47.6 us with every group masked
-// on whole workgroups, 31.7 with the branch, key-split workgroups and the
-// ranked order; fp16 [2, 10, 3952], ragged, 103 us on whole workgroups alone,
-// 90 on the mixed kind.
+// branch, whether keys have to be hidden. Ragged calls' other groups take the
+// plain step: fp16 [2, 10, 3952] 103 us on whole workgroups alone, 90 on the
+// mixed kind. Masked calls' keep the exact maximum (group_step, kHide): masked
+// causal fp16 [2, 16, 1500] 47.4 us with every group masked on whole
+// workgroups, 26.0 with the branch, key-split workgroups, the ranked order and
+// padding left out of the walk.
 // Whole and key-split workgroups share one kernel (one grid); each kind is
 // a separate instantiation of the body, so neither constrains the other's
 // register allocation. K ring then V ring in one array (the key-split merge
@@ -1787,13 +1795,14 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
     }
     if (mask_all) {
         // Masked calls, one kind per launch: key-split workgroups (64 rows)
-        // while they all fit three per CU under a causal limit, whose blocks
-        // are of unequal length, and while whole ones would not fill two per CU
+        // while whole ones would not fill two per CU under a causal limit, whose
+        // blocks are of unequal length, and while they all fit three per CU
         // without it; else whole ones. Measured, split against whole: causal
-        // [2, 16, 1500] 23.4 / 29.3 us, [4, 20, 1000] 30.7 / 31.3, [4, 20, 2000]
-        // (1280 units) 75.7 / 72.4; key mask alone [2, 16, 1500] 43 / 50,
-        // [4, 20, 1000] (640 units) 51.5 / 43.9.
-        if (units <= (p.causal ? slots : 2 * (int64_t)compute_units - 1)) {
+        // [2, 16, 1500] 26.0 / 34.0 us, [4, 20, 700] (480 units) 18.9 / 20.3,
+        // [4, 20, 1000] (640) 31.9 / 29.4; key mask alone [2, 16, 1500] (384)
+        // 34.1 / 37.8, [2, 16, 1800] (480) 57.3 / 50.4, [4, 16, 1000] (512)
+        // 30.7 / 26.4.
+        if (p.causal ? units <= 2 * (int64_t)compute_units : 2 * units <= slots) {
             p.whole_units = 0;
             p.split_units = (int32_t)(2 * units);
         }

@@ -87,3 +87,30 @@ def test_ragged_anchor_update(B, H, Sq, Sk):
         k[:, at] += k[:, at].sign() * 4
         check(q, k, v, H, "f16")
         check(q, k, v, H, "f16", causal=True)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("B,H,S", [(1, 2, 320), (2, 256, 256)])  # key-split and whole workgroups
+@pytest.mark.parametrize("top", [40, 70])
+def test_masked_largest_weight_is_exact(B, H, S, top, causal, dtype):
+    """Masked calls keep the running maximum exact, also in groups without a hidden key: keys 0-31
+    score 0, one later key a little above, the others far below, so every weight is a power of two or
+    zero and the output rounds once, at the end (half a unit, and 2^-17 for the fp32 arithmetic)."""
+    q, k, v = (torch.zeros(B, S, H * 64, device=DEV) for _ in range(3))
+    rows = torch.linspace(0.9, 1.1, S, device=DEV)
+    q[..., ::64] = 8 * rows[None, :, None]
+    k[:, 32:, ::64] = -60
+    k[:, top, ::64] = 3.4
+    v[:, :128] = 1 + torch.rand(B, 1, H * 64, device=DEV, generator=torch.Generator(device=DEV).manual_seed(S))
+    v[:, :32] *= 0.25
+    q, k, v = (x.to(DTYPES[dtype]) for x in (q, k, v))
+    mask = torch.ones(B, S, dtype=torch.int32, device=DEV)
+    mask[:, -1] = 0
+    got = sh.attention(q, k, v, H, causal=causal, key_mask=None if causal else mask)[:, 96:]
+    score = q[:, 96:, ::64].double() * k[:, top, None, ::64].double() / 8       # [B, rows, H]
+    weight = torch.exp(score).repeat_interleave(64, dim=-1)
+    ref = (weight * v[:, top, None].double() + 32 * v[:, 0, None].double()) / (weight + 32)
+    half_unit = torch.exp2(torch.floor(torch.log2(ref))) * UNIT[dtype]
+    excess = ((got.double() - ref).abs() - half_unit) / ref
+    assert excess.max().item() <= 2.0 ** -17, excess.max().item()
