@@ -296,14 +296,18 @@ KsplitTile ksplit_tile(const LinearParams& p, bool w_fp8, int compute_units) {
     // K = 2048, ~53 bytes a cycle), so the more CUs share it the better: [154,
     // 2048] x [2048, 2560] 60 tiles of 64 x 128 with producer waves 12.0 us,
     // 200 tiles of 32 x 64 8.8 us; x [1280, 2048] 10.9 -> 7.0 (32 x 32); [200, 640] x
-    // [640, 640] + bias + residual 6.7 -> 4.5; [308, 2048] x [2560, 2048] (64 x 64)
-    // 13.2 -> 13.1.
+    // [640, 640] + bias + residual 6.7 -> 4.5. 64 x 64 tiles for output
+    // projections of K >= 1024: x [1280, 1280] + bias + residual 600 rows 9.8 ->
+    // 8.4, 400 rows 8.7 -> 8.2 (level-2 cross sublayer of 400 rows 28.9 -> 24.9);
+    // without a residual they gain nothing ([308, 2048] x [2048, 2560] 12.6 both),
+    // and at K = 640 lose in the sublayer what they gain alone (1000 rows of
+    // level 1: alone 6.6 -> 6.3, sublayer 20.5 -> 21.2).
     // Projections without a residual only where the attention would run on
     // 16-row query blocks: beyond, the fused query projection +
     // cross-attention reproduces linear_kernel's accumulation order bit for bit.
     if (p.residual != nullptr || short_keys_16_row_blocks((int64_t)((p.m + 31) / 32) * ((p.n + 63) / 64), compute_units))
         for (KsplitTile t : {KsplitTile{1, 1}, KsplitTile{1, 2}, KsplitTile{2, 2}})
-            if (tasks_of(p, t) <= compute_units) return t;
+            if (tasks_of(p, t) <= compute_units && (t.mt == 1 || (p.residual != nullptr && p.k >= 1024))) return t;
     // Output projections (a residual) whose 64 x 160 tiles make one round that
     // fills at least 90 % of the CUs (the level-2 projections, 2048 x 1280: 256
     // tiles); with fewer tiles, or several per CU, the 64 x 128 kernels

@@ -229,7 +229,8 @@ def test_linear_k_split(M, N, K, bias):
                                    (200, 648, 640), (320, 2560, 576), (300, 1000, 1280)])
 @pytest.mark.parametrize("extras", [False, True])
 def test_linear_few_rows(M, N, K, extras):
-    """The 32 x 32, 32 x 64 and 64 x 64 tiles of the K-split kernel: edges of the tile, K below and above its ring."""
+    """The 32 x 32, 32 x 64 and 64 x 64 tiles of the K-split kernel and the rows beyond them: edges of the
+    tile, K below and above its ring."""
     g = torch.Generator(device=DEV).manual_seed(M + N)
     a = torch.randn(M, K, device=DEV, generator=g).half()
     w = (torch.randn(N, K, device=DEV, generator=g) / K ** 0.5).half()
