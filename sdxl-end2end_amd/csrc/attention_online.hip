@@ -18,7 +18,6 @@
 #include <stdint.h>
 
 #include "attention_kernels.hpp"
-#include "attention_row.hpp"
 
 namespace sdxl_hip {
 namespace {
@@ -28,8 +27,31 @@ constexpr int kMaxChannelsPerLane = kMaxHeadDim / 64;
 constexpr int kRowsPerBlock = 4;
 
 template <typename T>
+__device__ __forceinline__ float load_f(const T* p) {
+    return (float)(*p);
+}
+
+template <typename T>
+__device__ __forceinline__ void store_f(T* p, float v) {
+    *p = (T)v;
+}
+
+__device__ __forceinline__ float wave_max(float x) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x = fmaxf(x, __shfl_xor(x, off, 64));
+    return x;
+}
+
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+    return x;
+}
+
+template <typename T>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void online_attention_kernel(OnlineAttentionParams p) {
     __shared__ float q_lds[kRowsPerBlock][kMaxHeadDim];
+    const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int64_t rows = (int64_t)p.batch * p.heads * p.q_seq;
     const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + wave;
@@ -44,11 +66,60 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void online_attention_kernel(On
     const T* vb = (const T*)p.v + (int64_t)b * p.k_seq * p.v_row_stride + (int64_t)h * D;
     T* orow = (T*)p.o + ((int64_t)b * p.q_seq + query) * p.o_row_stride + (int64_t)h * D;
 
+    float* qs = q_lds[wave];
+    for (int d = lane; d < D; d += 64) qs[d] = load_f(qrow + d);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+    const int n_ch = (D + 63) >> 6;
+    float acc[kMaxChannelsPerLane];
+#pragma unroll
+    for (int t = 0; t < kMaxChannelsPerLane; ++t) acc[t] = 0.0f;
+    float m = -__builtin_inff();
+    float l = 0.0f;
+
     int n_keys = p.k_seq;
     if (p.causal) n_keys = n_keys < query + 1 ? n_keys : query + 1;
-    row_attention<T, kMaxChannelsPerLane>(qrow, kb, vb, orow, p.k_row_stride, p.v_row_stride,
-                                          p.key_mask != nullptr ? p.key_mask + (int64_t)b * p.k_seq : nullptr, n_keys, D, p.scale,
-                                          q_lds[wave]);
+
+    for (int k0 = 0; k0 < n_keys; k0 += 64) {
+        const int key = k0 + lane;
+        bool visible = key < n_keys;
+        if (visible && p.key_mask != nullptr) visible = p.key_mask[(int64_t)b * p.k_seq + key] != 0;
+        float s = -__builtin_inff();
+        if (visible) {
+            const T* krow = kb + (int64_t)key * p.k_row_stride;
+            float dot = 0.0f;
+            for (int d = 0; d < D; ++d) dot += qs[d] * load_f(krow + d);
+            s = dot * p.scale;
+        }
+        const float m_new = fmaxf(m, wave_max(s));
+        if (m_new == -__builtin_inff()) continue;  // nothing visible yet
+        const float alpha = m == -__builtin_inff() ? 0.0f : expf(m - m_new);
+        const float pr = visible ? expf(s - m_new) : 0.0f;
+        l = l * alpha + wave_sum(pr);
+        m = m_new;
+        const int chunk = n_keys - k0 < 64 ? n_keys - k0 : 64;
+#pragma unroll
+        for (int t = 0; t < kMaxChannelsPerLane; ++t) {
+            if (t < n_ch) acc[t] *= alpha;
+        }
+        for (int j = 0; j < chunk; ++j) {
+            const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pr), j));
+            const T* vrow = vb + (int64_t)(k0 + j) * p.v_row_stride;
+#pragma unroll
+            for (int t = 0; t < kMaxChannelsPerLane; ++t) {
+                const int d = lane + 64 * t;
+                if (t < n_ch && d < D) acc[t] += pj * load_f(vrow + d);
+            }
+        }
+    }
+    const float inv = 1.0f / fmaxf(l, 1.0e-20f);
+#pragma unroll
+    for (int t = 0; t < kMaxChannelsPerLane; ++t) {
+        const int d = lane + 64 * t;
+        if (t < n_ch && d < D) store_f(orow + d, acc[t] * inv);
+    }
 }
 
 }  // namespace

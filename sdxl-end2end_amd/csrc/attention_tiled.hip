@@ -35,14 +35,13 @@
 // LDS rows are 64-dim panels of 128 bytes, 16-byte chunks XOR-swizzled by row.
 //
 // Values that planes cannot carry (infinities, NaN, fp32 above the largest
-// bf16) leave NaN in the results; a query block with any runs the per-row
-// kernel's code instead (attention_row.hpp).
+// bf16) leave NaN in the results; a query block with any starts over in plain
+// fp32, its rows dealt to the waves of its key groups (redo_rows).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "attention_kernels.hpp"
 #include "attention_planes.hpp"
-#include "attention_row.hpp"
 
 namespace sdxl_hip {
 namespace {
@@ -52,6 +51,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef __attribute__((address_space(3))) i16x8 lds_i16x8;
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 
 constexpr int kKeys = 32;                       // keys per sub-tile
 constexpr int kPanelBytes = kKeys * 128;        // 32 rows of 64 16-bit values
@@ -60,6 +60,16 @@ __device__ __forceinline__ int rev3(int x) { return ((x & 1) << 2) | (x & 2) | (
 __device__ __forceinline__ int swz(int row) { return rev3((row >> 1) & 7); }
 __device__ __forceinline__ float xhalf_max(float x) { return fmaxf(x, __shfl_xor(x, 32, 64)); }
 __device__ __forceinline__ float xhalf_sum(float x) { return x + __shfl_xor(x, 32, 64); }
+__device__ __forceinline__ float wave_max(float x) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x = fmaxf(x, __shfl_xor(x, off, 64));
+    return x;
+}
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+    return x;
+}
 
 template <typename T> struct Planes;
 template <> struct Planes<float> { static constexpr int in = 3, prob = 3; static constexpr bool f16 = false; static constexpr float shift = 0.0f; };
@@ -125,11 +135,102 @@ __device__ __forceinline__ void zero_past(u32x4 (&pl)[kN], int n) {
         for (int e = 0; e < 4; ++e) pl[i][e] = 2 * e >= n ? 0u : 2 * e + 1 >= n ? pl[i][e] & 0xFFFFu : pl[i][e];
 }
 
-// A row in plain fp32 (out of line: it leaves the tiled kernel's registers alone).
-template <typename T>
-__device__ __attribute__((noinline)) void plain_row(const T* q, const T* k, const T* v, T* o, int64_t k_stride, int64_t v_stride,
-                                                    const int32_t* mask, int n_keys, int dim, float scale, float* qs) {
-    row_attention<T, 3>(q, k, v, o, k_stride, v_stride, mask, n_keys, dim, scale, qs);
+// kRedoRows query rows in plain fp32 by one wave, for the blocks whose values
+// planes cannot carry: the per-row kernel's steps (attention_online.hip: chunks
+// of 64 keys, one key per lane for the scores, one output channel per lane for
+// the output), with each K and V value loaded once for all of the rows. In line
+// and small, so that it takes no more registers than the kernel around it.
+// A NaN in K, so every block here: FP32 [1, 20, 1024, 64] 0.73 ms, fp16 [2, 8, 1000,
+// 80] 0.73 (1.94 and 1.67 on the per-row kernel, 8.3 and 11.6 with one row at a
+// time by the first wave of a query block alone). q and o point at the first of
+// the rows; qs: kRedoRows * dim floats of LDS of the wave's own.
+template <typename T, int kRedoRows>
+__device__ __forceinline__ void redo_rows(const T* q, const T* k, const T* v, T* o, int64_t q_stride, int64_t k_stride,
+                                                    int64_t v_stride, int64_t o_stride, const int32_t* mask, int rows, int first_row,
+                                                    int k_seq, bool causal, int dim, float scale, lds_f32x4* qs) {
+    constexpr int kChannels = 3;  // dim <= 160
+    const int lane = threadIdx.x & 63;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int d = lane; d < dim; d += 64) {
+#pragma unroll
+        for (int h = 0; h < kRedoRows / 4; ++h) {
+            f32x4 x;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = (float)q[min(4 * h + r, rows - 1) * q_stride + d];
+            qs[(kRedoRows / 4) * d + h] = x;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+    float acc[kRedoRows][kChannels], m[kRedoRows], l[kRedoRows];
+#pragma unroll
+    for (int r = 0; r < kRedoRows; ++r) {
+        m[r] = -__builtin_inff();
+        l[r] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < kChannels; ++t) acc[r][t] = 0.0f;
+    }
+    const int n_keys = causal ? min(k_seq, first_row + rows) : k_seq;
+#pragma unroll 1
+    for (int k0 = 0; k0 < n_keys; k0 += 64) {
+        const int key = min(k0 + lane, k_seq - 1);
+        const bool shown = k0 + lane < n_keys && (mask == nullptr || mask[key] != 0);
+        const T* krow = k + (int64_t)key * k_stride;
+        float p[kRedoRows];
+#pragma unroll
+        for (int r = 0; r < kRedoRows; ++r) p[r] = 0.0f;
+#pragma unroll 4
+        for (int d = 0; d < dim; ++d) {
+            const float x = (float)krow[d];
+#pragma unroll
+            for (int h = 0; h < kRedoRows / 4; ++h) {
+                const f32x4 y = qs[(kRedoRows / 4) * d + h];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[4 * h + r] += y[r] * x;
+            }
+        }
+        int chunk[kRedoRows];  // keys of the chunk that reach the row
+#pragma unroll
+        for (int r = 0; r < kRedoRows; ++r) {
+            const int row_keys = causal ? min(k_seq, first_row + r + 1) : k_seq;
+            const bool visible = shown && key < row_keys;
+            const float s = visible ? p[r] * scale : -__builtin_inff();
+            const float m_new = fmaxf(m[r], wave_max(s));
+            const bool none = m_new == -__builtin_inff();  // no finite score yet: the chunk is left out
+            const float alpha = m[r] == -__builtin_inff() ? 0.0f : expf(m[r] - m_new);
+            p[r] = visible && !none ? expf(s - m_new) : 0.0f;
+            l[r] = l[r] * alpha + wave_sum(p[r]);
+            m[r] = m_new;
+            chunk[r] = none ? 0 : __builtin_amdgcn_readfirstlane(min(64, row_keys - k0));
+#pragma unroll
+            for (int t = 0; t < kChannels; ++t) acc[r][t] *= alpha;
+        }
+        const int n = min(64, n_keys - k0);
+#pragma unroll 4
+        for (int j = 0; j < n; ++j) {
+            const T* vrow = v + (int64_t)(k0 + j) * v_stride;
+            float x[kChannels];
+#pragma unroll
+            for (int t = 0; t < kChannels; ++t) x[t] = (float)vrow[min(lane + 64 * t, dim - 1)];
+#pragma unroll
+            for (int r = 0; r < kRedoRows; ++r) {
+                const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p[r]), j));
+#pragma unroll
+                for (int t = 0; t < kChannels; ++t)
+                    if (j < chunk[r]) acc[r][t] += pj * x[t];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kRedoRows; ++r) {
+        const float inv = 1.0f / fmaxf(l[r], 1.0e-20f);
+#pragma unroll
+        for (int t = 0; t < kChannels; ++t)
+            if (r < rows && lane + 64 * t < dim) o[r * o_stride + lane + 64 * t] = (T)(acc[r][t] * inv);
+    }
 }
 
 constexpr int tiled_panels(int dp) { return (dp + 63) / 64; }
@@ -154,7 +255,10 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
     constexpr int kMergeBytes = (4 - kQB) * kMergeFloats * 64 * 4;
     constexpr int kLdsBytes = 2 * kKS * kSub > kMergeBytes ? 2 * kKS * kSub : kMergeBytes;
     static_assert(kLdsBytes <= 160 * 1024 - 64, "LDS");
+    constexpr int kRedoRows = sizeof(T) == 4 || kDp > 64 ? 8 : 4;  // as many as the kernel's registers hold
+    static_assert(kRedoRows % 4 == 0 && 4 * kRedoRows * kDp * 4 <= kLdsBytes, "queries of redo_rows");
     __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];
+    __shared__ int special[kQB];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -381,9 +485,8 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
             mine[(16 * kTiles + 1) * 64] = l_tot;
         }
         __syncthreads();
-        if (kg > 0) return;
 #pragma unroll 1
-        for (int g = 1; g < kKS; ++g) {
+        for (int g = 1; g < (kg == 0 ? kKS : 0); ++g) {
             const float* part = park + g * (kMergeFloats * 64);
             const float m1 = part[16 * kTiles * 64];
             const float mx = fmaxf(m_run, m1);
@@ -401,7 +504,7 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
     const float inv = 1.0f / fmaxf(l_tot, 1.0e-20f);
     // Planes turn an infinity, a NaN or an FP32 value above the largest bf16
     // into a NaN, which reaches every score or output that it meets: a query
-    // block with one (or whose results overflow) starts over in plain fp32.
+    // block with one (or whose results overflow) starts over in fp32.
     float bad = l_tot;
 #pragma unroll
     for (int t = 0; t < kTiles; ++t)
@@ -410,15 +513,17 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
             acc[t][i] *= inv;
             bad = __builtin_fmaf(acc[t][i], 0.0f, bad);
         }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad != bad) != 0, 0)) {
-        __shared__ float row_q[4][kDp];
+    if (kg == 0) special[wave / kKS] = __builtin_amdgcn_ballot_w64(bad != bad) != 0;
+    __syncthreads();  // also: nobody reads the tiles or the parked sums any more
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(special[wave / kKS]) != 0, 0)) {
 #pragma unroll 1
-        for (int r = 0; r < 32 && q0 + r < p.q_seq; ++r)
-            plain_row<T>(qbase + (int64_t)(q0 + r) * p.q_row_stride, kbase, vbase, obase + (int64_t)(q0 + r) * p.o_row_stride,
-                         p.k_row_stride, p.v_row_stride, p.key_mask != nullptr ? p.key_mask + (int64_t)b * p.k_seq : nullptr,
-                         p.causal ? min(p.k_seq, q0 + r + 1) : p.k_seq, D, p.scale, row_q[wave]);
+        for (int r = q0 + kRedoRows * kg; r < min(q0 + 32, p.q_seq); r += kRedoRows * kKS)
+            redo_rows<T, kRedoRows>(qbase + (int64_t)r * p.q_row_stride, kbase, vbase, obase + (int64_t)r * p.o_row_stride, p.q_row_stride,
+                         p.k_row_stride, p.v_row_stride, p.o_row_stride, p.key_mask != nullptr ? p.key_mask + (int64_t)b * p.k_seq : nullptr,
+                         min(kRedoRows, p.q_seq - r), r, p.k_seq, p.causal != 0, D, p.scale, (lds_f32x4*)lds + wave * (kRedoRows / 4 * kDp));
         return;
     }
+    if (kg > 0) return;
     if (my_query >= p.q_seq) return;
     T* orow = obase + (int64_t)my_query * p.o_row_stride;
 #pragma unroll

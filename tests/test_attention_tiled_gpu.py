@@ -137,3 +137,22 @@ def test_tiled_large_logits():
 def test_tiled_limit_of_the_head_dimension(D):
     q, k, v = tensors(13, 1, 2, 40, 50, D, "f32")
     check(sh.attention(q, k, v, 2), reference(q, k, v, 2), "f32")
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal", [
+    (1, 2, 70, 70, 40, True), (1, 1, 131, 131, 160, True), (2, 3, 90, 200, 33, True), (2, 2, 100, 100, 7, False),
+    (2, 40, 1000, 70, 40, False), (1, 33, 1000, 150, 56, True)])  # one and two key groups on full grids
+def test_tiled_special_values_reach_their_rows_alone(B, H, Sq, Sk, D, causal, where, value, dtype):
+    """Rows that a causal limit keeps away from an infinity or a NaN stay finite; every other row as on
+    the per-row kernel, on each workgroup form, also with rows left over from the groups that start over."""
+    q, k, v = tensors(Sq + D, B, H, Sq, Sk, D, dtype)
+    at = 37
+    {"q": q, "k": k, "v": v}[where][0, at, D + 3 if H > 1 else 3] = value
+    got = sh.attention(q, k, v, H, causal=causal).float()
+    ref = sh.attention(q, k, v, H, causal=causal, backend=sh.WARP_ONLINE).float()
+    torch.testing.assert_close(got, ref, rtol=2.0 ** -7 if dtype == "bf16" else 2e-3, atol=1e-3, equal_nan=True)
+    if causal and where != "q":
+        assert got[0, :at].isfinite().all()
