@@ -87,46 +87,124 @@ __device__ __forceinline__ float group_sum(float x) {
     return x;
 }
 
-// 64 kN dims of one output row in plain fp32 by a wave, for the calls whose
-// values planes cannot carry: as the per-row kernel, a NaN score making the
-// row NaN. v and o point at the first of those dims.
-template <int kN>
-__device__ __attribute__((noinline)) void plain_row(const float* q, const float* k, const float* v, float* o, int64_t k_stride,
-                                                    int64_t v_stride, int k_seq, float scale) {
+// Whether every one of the workgroup's queries, or any key, holds a NaN: all of
+// the workgroup's results are NaN then, as they stand. flags: two zeros in LDS.
+__device__ __forceinline__ bool all_rows_nan(const float* q, const float* k, int64_t q_stride, int64_t k_stride, int rows, int k_seq,
+                                             volatile __attribute__((address_space(3))) int* flags) {
     const int lane = threadIdx.x & 63;
-    float acc[kN];
-    for (int i = 0; i < kN; ++i) acc[i] = 0.0f;
-    float m = -__builtin_inff(), l = 0.0f;
-    bool nan = false;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto row_nan = [&](const float* row) __attribute__((always_inline)) {
+        const f32x4 x = *(const f32x4*)(row + 4 * lane), y = *(const f32x4*)(row + 256 + 4 * lane);
+        return __builtin_isunordered(x[0], x[1]) || __builtin_isunordered(x[2], x[3]) || __builtin_isunordered(y[0], y[1]) ||
+               __builtin_isunordered(y[2], y[3]);
+    };
 #pragma unroll 1
-    for (int k0 = 0; k0 < k_seq; k0 += 64) {
-        const float* key = k + (int64_t)min(k0 + lane, k_seq - 1) * k_stride;
-        float s = 0.0f;
+    for (int r = wave; r < rows; r += kWaves)
+        if (__builtin_amdgcn_ballot_w64(row_nan(q + (int64_t)r * q_stride)) == 0) flags[0] = 1;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(flags[0]) == 0) return true;
 #pragma unroll 1
-        for (int d = 0; d < kDim; ++d) s += q[d] * key[d];
-        s *= scale;
-        if (k0 + lane >= k_seq) s = -__builtin_inff();
-        nan = nan || __builtin_amdgcn_ballot_w64(s != s) != 0;
-        float mx = s;
-        for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-        const float m_new = fmaxf(m, mx);
-        if (m_new == -__builtin_inff()) continue;
+    for (int key0 = 8 * wave; key0 < k_seq && flags[1] == 0; key0 += 8 * kWaves) {
+        bool nan = false;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) nan = row_nan(k + (int64_t)min(key0 + r, k_seq - 1) * k_stride) || nan;
+        if (__builtin_amdgcn_ballot_w64(nan) != 0) flags[1] = 1;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(flags[1]) != 0;
+}
+
+// The output of 32 queries from the start on v_mfma_f32_32x32x2, for calls whose
+// values planes cannot carry: the same split over waves and exchange of
+// partials, without the pipeline. A NaN score makes its row NaN. q and o point
+// at the first query of the rows left, v and o at the wave's first output dim.
+// An infinity in K: 16384 tokens 10.7 ms in all (fp32 matrix instructions
+// throughout took 5.0, plain rows by a wave each 282), 4096 tokens 1.16 (0.40,
+// 35); a NaN in K, by all_rows_nan, 2.7 and 0.37.
+template <int kDT>
+__device__ __forceinline__ void redo_block(const float* q, const float* k, const float* v, float* o, int64_t q_stride, int64_t k_stride,
+                                           int64_t v_stride, int64_t o_stride, int rows, int k_seq, float scale, lds_f32x4* part) {
+    const int lane = threadIdx.x & 63, hf = lane >> 5, col = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    f32x4 qx[kSlice / 8], kx[kSlice / 8];  // lane holds query or key col, dims 8 n + 4 hf .. +3 of the slice
+    const float* qrow = q + (int64_t)min(col, rows - 1) * q_stride + kSlice * wave + 4 * hf;
+    auto load_k = [&](int key0) __attribute__((always_inline)) {
+        const float* krow = k + (int64_t)min(key0 + col, k_seq - 1) * k_stride + kSlice * wave + 4 * hf;
+#pragma unroll
+        for (int n = 0; n < kSlice / 8; ++n) kx[n] = *(const f32x4*)(krow + 8 * n);
+    };
+#pragma unroll
+    for (int n = 0; n < kSlice / 8; ++n) qx[n] = *(const f32x4*)(qrow + 8 * n);
+    load_k(0);
+    f32x16 acc[kDT];
+#pragma unroll
+    for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[dt][i] = 0.0f;
+    float m = -__builtin_inff(), l = 0.0f;  // l: this lane's half of the keys
+#pragma unroll 1
+    for (int key0 = 0; key0 < k_seq; key0 += kKeys) {
+        f32x16 s;  // element i: key 8 (i / 4) + 4 hf + i % 4
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+        for (int n = 0; n < kSlice / 8; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[n][i], qx[n][i], s, 0, 0, 0);
+        // the next block's K and this one's V arrive during the exchange
+        load_k(key0 + kKeys);
+        float vx[16][kDT];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float* vrow = v + (int64_t)min(key0 + 8 * (i >> 2) + 4 * hf + (i & 3), k_seq - 1) * v_stride + col;
+#pragma unroll
+            for (int dt = 0; dt < kDT; ++dt) vx[i][dt] = vrow[32 * dt];
+        }
+        __syncthreads();  // the last block's partials are used
+#pragma unroll
+        for (int u = 0; u < 4; ++u) part[(wave * 4 + u) * 64 + lane] = f32x4{s[4 * u], s[4 * u + 1], s[4 * u + 2], s[4 * u + 3]};
+        __syncthreads();
+        float mx = -__builtin_inff();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            f32x4 x = part[u * 64 + lane];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) x += part[(w * 4 + u) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                s[4 * u + r] = key0 + 8 * u + 4 * hf + r < k_seq ? x[r] * scale : -__builtin_inff();
+                mx = fmaxf(mx, s[4 * u + r]);
+            }
+        }
+        const float m_new = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));
         const float alpha = m == -__builtin_inff() ? 0.0f : expf(m - m_new);
-        const float pr = k0 + lane < k_seq ? expf(s - m_new) : 0.0f;
-        float sum = pr;
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-        l = l * alpha + sum;
         m = m_new;
-        for (int i = 0; i < kN; ++i) acc[i] *= alpha;
-        const int n = min(64, k_seq - k0);
-#pragma unroll 1
-        for (int j = 0; j < n; ++j) {
-            const float pj = __shfl(pr, j, 64);
-            for (int i = 0; i < kN; ++i) acc[i] += pj * v[(int64_t)(k0 + j) * v_stride + lane + 64 * i];
+        l *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
+        // O^T += V^T P^T; keys that do not exist count as zero rows
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            // -inf weighs nothing, also while there is no finite score; NaN stays
+            const float pr = s[i] == -__builtin_inff() ? 0.0f : expf(s[i] - m);
+            l += pr;
+            const bool in = key0 + 8 * (i >> 2) + 4 * hf + (i & 3) < k_seq;
+#pragma unroll
+            for (int dt = 0; dt < kDT; ++dt) acc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? vx[i][dt] : 0.0f, pr, acc[dt], 0, 0, 0);
         }
     }
-    const float inv = nan ? __builtin_nanf("") : 1.0f / fmaxf(l, 1.0e-20f);
-    for (int i = 0; i < kN; ++i) o[lane + 64 * i] = acc[i] * inv;
+    const float total = l + __shfl_xor(l, 32, 64);
+    const float inv = total != total ? total : 1.0f / fmaxf(total, 1.0e-20f);
+    if (col >= rows) return;
+    float* row = o + (int64_t)col * o_stride + 4 * hf;
+#pragma unroll
+    for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            *(f32x4*)(row + 32 * dt + 8 * u) = f32x4{acc[dt][4 * u] * inv, acc[dt][4 * u + 1] * inv, acc[dt][4 * u + 2] * inv,
+                                                     acc[dt][4 * u + 3] * inv};
 }
 
 template <int kN> struct PerLane;
@@ -150,7 +228,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     __shared__ __attribute__((aligned(16))) char prob[kProbBytes];  // [tile][16-key half][plane][64] x 16 bytes
     __shared__ float scale_o[32 * kQT];
     __shared__ float total[32 * kQT];
-    __shared__ int special;
+    __shared__ int special, seen[2];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -169,7 +247,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     const uint32_t k_stride_b = (uint32_t)(p.k_row_stride * 4), v_stride_b = (uint32_t)(p.v_row_stride * 4);
     const int n_blocks = (p.k_seq + kKeys - 1) / kKeys;
 
-    if (threadIdx.x == 0) special = 0;
+    if (threadIdx.x == 0) special = seen[0] = seen[1] = 0;
     __syncthreads();
 
     // Block t is rows first_row(t) .. +31: a last block that k_seq does not fill
@@ -548,7 +626,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     __syncthreads();
     // Planes turn an infinity, a NaN or an FP32 value above the largest bf16
     // into a NaN, which reaches every score or output that it meets: such
-    // workgroups (and those whose results overflow) start over in plain fp32.
+    // workgroups (and those whose results overflow) start over in fp32, unless
+    // a NaN has decided all of their results.
     float bad = 0.0f;
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt) {
@@ -563,15 +642,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     }
     if (bad != bad) atomicOr(&special, 1);
     __syncthreads();
-    if (__builtin_expect(__builtin_amdgcn_readfirstlane(special) != 0, 0)) {
+    bool redo = __builtin_amdgcn_readfirstlane(special) != 0;
+    if (__builtin_expect(redo, 0))
+        redo = !all_rows_nan(qhead + (int64_t)q0 * p.q_row_stride, khead, p.q_row_stride, p.k_row_stride, min(32 * kQT, p.q_seq - q0),
+                             p.k_seq, (__attribute__((address_space(3))) int*)seen);
+    if (__builtin_expect(redo, 0)) {
 #pragma unroll 1
-        for (int r = wave; r < 32 * kQT; r += kWaves)
-            if (q0 + r < p.q_seq) {
-                const int first = (kDim / kParts) * out_part;
-                plain_row<kDim / kParts / 64>(qhead + (int64_t)(q0 + r) * p.q_row_stride, khead, vhead + first,
-                                              ohead + (int64_t)(q0 + r) * p.o_row_stride + first, p.k_row_stride, p.v_row_stride,
-                                              p.k_seq, p.scale);
-            }
+        for (int first = q0; first < min(q0 + 32 * kQT, p.q_seq); first += 32)
+            redo_block<kDT>(qhead + (int64_t)first * p.q_row_stride, khead, vhead + out_dim, ohead + (int64_t)first * p.o_row_stride + out_dim,
+                            p.q_row_stride, p.k_row_stride, p.v_row_stride, p.o_row_stride, min(32, p.q_seq - first), p.k_seq, p.scale,
+                            (lds_f32x4*)part);
         return;
     }
     // lane holds tile rows m = 8u + 4hf + r of query col: dims kDT m + dt

@@ -156,3 +156,26 @@ def test_tiled_special_values_reach_their_rows_alone(B, H, Sq, Sk, D, causal, wh
     torch.testing.assert_close(got, ref, rtol=2.0 ** -7 if dtype == "bf16" else 2e-3, atol=1e-3, equal_nan=True)
     if causal and where != "q":
         assert got[0, :at].isfinite().all()
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 9, 950, 70), (1, 6, 1000, 70), (1, 1, 70, 300), (1, 9, 950, 32)])
+@pytest.mark.parametrize("where", ["q", "k", "v", "all"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.402e38])
+def test_d512_special_values_on_every_form(B, H, Sq, Sk, where, value):
+    """As test_d512_values_planes_cannot_carry, on 64 queries per workgroup, on 32 with all output dims,
+    and on two workgroups per query block; and with every query of a block of rows special."""
+    q, k, v = tensors(Sq + Sk, B, H, Sq, Sk, 512, "f32")
+    h = H - 1
+    if where == "all":
+        q[0, :64, 512 * h + 5] = value
+        rows = range(0, 64)
+    else:
+        {"q": q, "k": k, "v": v}[where][0, 27, 512 * h + 300] = value
+        rows = [27] if where == "q" else []
+    got = sh.attention(q, k, v, H)
+    ref = sh.attention(q, k, v, H, backend=sh.WARP_ONLINE)
+    if value != value:
+        for r in rows:  # the per-row kernel takes such a row's keys for hidden
+            assert got[0, r, 512 * h:].isnan().all()
+            got[0, r, 512 * h:] = ref[0, r, 512 * h:]
+    torch.testing.assert_close(got, ref, rtol=2e-3, atol=1e-3, equal_nan=True)
