@@ -34,18 +34,31 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 __device__ __forceinline__ float lo_bf16(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
 __device__ __forceinline__ float hi_bf16(uint32_t v) { return __builtin_bit_cast(float, v & 0xFFFF0000u); }
 
-// Two values as kN planes: bf16 planes (exact for kN = 3) or two fp16 planes.
+// a less the low (kHi: high) fp16 value of h, in one instruction.
+template <bool kHi>
+__device__ __forceinline__ float less_f16(float a, uint32_t h) {
+    float r;
+    if constexpr (kHi) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(a));
+    else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(a));
+    return r;
+}
+
+// Two values as kN bf16 or fp16 planes, each holding what the ones before it
+// left. fp16 planes before the last are truncated, two values in one
+// instruction.
 template <int kN, bool kF16>
 __device__ __forceinline__ void split2(float a, float b, uint32_t (&out)[kN]) {
-    if constexpr (kF16) {
-        static_assert(kN == 2);
-        const f16x2 h = {(_Float16)a, (_Float16)b};
-        const f16x2 l = {(_Float16)(a - (float)h[0]), (_Float16)(b - (float)h[1])};
-        out[0] = __builtin_bit_cast(uint32_t, h);
-        out[1] = __builtin_bit_cast(uint32_t, l);
-    } else {
 #pragma unroll
-        for (int i = 0; i < kN; ++i) {
+    for (int i = 0; i < kN; ++i) {
+        if constexpr (kF16) {
+            if (i + 1 == kN) {
+                out[i] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
+            } else {
+                out[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+                a = less_f16<false>(a, out[i]);
+                b = less_f16<true>(b, out[i]);
+            }
+        } else {
             out[i] = pack_bf16(a, b);
             if (i + 1 < kN) {
                 a -= lo_bf16(out[i]);

@@ -10,8 +10,10 @@
 // at least 2^-17 of it (hh, hm, mh, mm, hl, lh); the dropped ones weigh 2^-26,
 // below an fp32 rounding. fp16 and bf16 inputs are one plane, exact. The
 // probabilities, fp32 in the per-row kernel, keep their bits as planes too:
-// three bf16 planes for fp32 and bf16 calls, two fp16 planes (22 bits, scaled
-// by 2^12 so that small ones keep theirs) for fp16 calls. All sums are fp32.
+// three bf16 planes for fp32 and bf16 calls, three fp16 planes scaled by 2^15
+// for fp16 calls: all 24 bits of those from 2^-16 of the row's largest on, below
+// within 2^-40 of it, which times the largest fp16 value is the smallest one
+// ([2, 8, 1000, 80] 30.1 us; two planes, 22 bits, took 27.3). All sums are fp32.
 //
 // Work split: a workgroup = 4 waves = 4 / kKS blocks of 32 queries x kKS key
 // groups. Per stage kKS sub-tiles of 32 keys are loaded (into registers, one
@@ -23,7 +25,7 @@
 //
 // Measured (graph replay): FP32 [1, 20, 1024, 64] 1943 us on the per-row kernel,
 // 58 us here (92 TFLOP/s; the fp32 matrix cores' peak is 157); FP32
-// [2, 8, 1000, 160] 91 us, fp16 [2, 8, 1000, 80] 1676 -> 28.5 us. Against 64 bits
+// [2, 8, 1000, 160] 91 us, fp16 [2, 8, 1000, 80] 1676 -> 30.1 us. Against 64 bits
 // the FP32 result is closer than the per-row kernel's (4.1e-7 against 6.4e-7 of
 // the output's norm at 1024 keys). Per wave and sub-tile 48 MFMAs (1536 cycles)
 // meet ~400 other vector instructions (~1600 cycles: the split of the stage's
@@ -74,7 +76,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 template <typename T> struct Planes;
 template <> struct Planes<float> { static constexpr int in = 3, prob = 3; static constexpr bool f16 = false; static constexpr float shift = 0.0f; };
 template <> struct Planes<__bf16> { static constexpr int in = 1, prob = 3; static constexpr bool f16 = false; static constexpr float shift = 0.0f; };
-template <> struct Planes<_Float16> { static constexpr int in = 1, prob = 2; static constexpr bool f16 = true; static constexpr float shift = 12.0f; };
+template <> struct Planes<_Float16> { static constexpr int in = 1, prob = 3; static constexpr bool f16 = true; static constexpr float shift = 15.0f; };
 
 // Eight values of a row as loaded (fp32: two registers of four; 16-bit: one).
 template <typename T> struct Raw { u32x4 v[sizeof(T) == 4 ? 2 : 1]; };
@@ -146,8 +148,8 @@ __device__ __forceinline__ void zero_past(u32x4 (&pl)[kN], int n) {
 // the rows; qs: kRedoRows * dim floats of LDS of the wave's own.
 template <typename T, int kRedoRows>
 __device__ __forceinline__ void redo_rows(const T* q, const T* k, const T* v, T* o, int64_t q_stride, int64_t k_stride,
-                                                    int64_t v_stride, int64_t o_stride, const int32_t* mask, int rows, int first_row,
-                                                    int k_seq, bool causal, int dim, float scale, lds_f32x4* qs) {
+                                          int64_t v_stride, int64_t o_stride, const int32_t* mask, int rows, int first_row,
+                                          int k_seq, bool causal, int dim, float scale, lds_f32x4* qs) {
     constexpr int kChannels = 3;  // dim <= 160
     const int lane = threadIdx.x & 63;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

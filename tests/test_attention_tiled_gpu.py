@@ -179,3 +179,25 @@ def test_d512_special_values_on_every_form(B, H, Sq, Sk, where, value):
             assert got[0, r, 512 * h:].isnan().all()
             got[0, r, 512 * h:] = ref[0, r, 512 * h:]
     torch.testing.assert_close(got, ref, rtol=2e-3, atol=1e-3, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("D", [80, 33])
+def test_tiled_small_probabilities_keep_their_bits(D, dtype):
+    """Two visible keys, one of weight ~1 with V = 0, one of weight exp(-a), a = 11 .. 24, with the largest
+    fp16 value: the output shows the small weight's own accuracy. fp16 planes hold it within 2^-40 of the
+    largest weight."""
+    B, H, S = 1, 2, 96
+    q, k, v = (torch.zeros(B, S, H * D, device=DEV, dtype=DTYPES[dtype]) for _ in range(3))
+    q[..., ::D] = torch.linspace(11, 24, S, device=DEV).to(DTYPES[dtype])[None, :, None]
+    k[..., ::D] = -60
+    k[:, 0, ::D] = 0
+    k[:, 5, ::D] = -1  # in the first key's sub-tile, so under its maximum
+    v[:, 5] = 65504 if dtype == "f16" else 65280
+    got = sh.attention(q, k, v, H, scale=1.0).double()
+    w = torch.exp(-q[..., ::D].double()).repeat_interleave(D, dim=-1)
+    ref = w / (1 + w) * v[0, 5, 0].double()
+    # a fp32 argument of exp2 up to 35 moves the weight by 35 ln 2 * 2^-24 < 2^-18
+    bound = ref * (OUT_ROUNDING[dtype] + 2.0 ** -18) + (2.0 ** -25 + 2.0 ** -24 if dtype == "f16" else 0)
+    worst = ((got - ref).abs() / bound).max().item()
+    assert worst <= 1, worst
