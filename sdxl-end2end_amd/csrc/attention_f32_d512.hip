@@ -8,8 +8,8 @@
 // (softmax with a running maximum, output divided by max(sum, 1e-20));
 // non-causal, unmasked calls with 16-byte aligned rows.
 //
-// Arithmetic: operands are split exactly into three bf16 planes and a product
-// is six plane products on the bf16 matrix cores (attention_planes.hpp), 2.7x
+// Arithmetic: operands are split into three bf16 planes and a product is six
+// plane products on the bf16 matrix cores (attention_planes.hpp), 2.7x
 // the fp32 matrix cores' rate; all sums are fp32.
 //
 // Work split: a workgroup = 8 waves = 32 kQT queries of one (batch, head);
@@ -304,6 +304,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
 
     // Q planes: lane holds query q0 + 32 qt + col, dims 16 ks + 8 hf .. +7.
     i16x8 qop[kQT][kSteps][kRegPlanes];
+    const float c = p.scale * 1.4426950408889634f;  // scores to log2 units
+    uint32_t q_smallest = ~0u;
+    float q_largest = 0.0f;
     char* const qlow_mine = qlow + (kQT == 2 ? wave * kQT * (kSteps + 1) * 1024 : 0) + lane * 16;
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt) {
@@ -314,6 +317,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const f32x2 x = *(const f32x2*)(row + 16 * ks + 2 * i);
+                q_smallest = min(q_smallest, min(nonzero_magnitude(x[0]), nonzero_magnitude(x[1])));
+                q_largest = fmaxf(q_largest, fmaxf(fabsf(x[0]), fabsf(x[1])));
                 uint32_t w[3];
                 split2<3, false>(x[0], x[1], w);
 #pragma unroll
@@ -328,6 +333,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+
+    if (!planes_carry_queries(q_smallest, q_largest, c)) special = 1;
 
     f32x16 o[kQT][kDT];  // [tile][dt]: dims kDT m + dt of the slice, m the tile row
 #pragma unroll
@@ -449,7 +456,6 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     const char* const part_mine = part + (st * 4 + su) * 1024 + (32 * sh + (sq ^ (2 * (2 * su + sh)))) * 16 + 4 * sr;
     // B operand of P.V: 16-key half ss, lane (hf', query): keys 16 ss + 8 hf' + e
     char* const prob_mine = prob + (st * 2 + (su >> 1)) * 3 * 1024 + (32 * (su & 1) + sq) * 16 + 8 * sh + 2 * sr;
-    const float c = p.scale * 1.4426950408889634f;  // scores to log2 units
     float m_run = -__builtin_inff(), l_run = 0.0f;  // of query sq; this lane's part of the sum
 
     float sc[kPer];
@@ -485,7 +491,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
         float pr[kPer], sum = 0.0f;
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
-            pr[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c, -m_new));
+            pr[i] = 65536.0f * __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c, -m_new));  // small ones keep their planes
             sum += pr[i];
         }
         l_run = l_run * alpha + sum;
@@ -626,9 +632,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
     __syncthreads();
     // Planes turn an infinity, a NaN or an FP32 value above the largest bf16
     // into a NaN, which reaches every score or output that it meets: such
-    // workgroups (and those whose results overflow) start over in fp32, unless
-    // a NaN has decided all of their results.
+    // workgroups (and those whose results overflow, or are so small that planes
+    // may have lost bits of them) start over in fp32, unless a NaN has decided
+    // all of their results.
     float bad = 0.0f;
+    uint32_t smallest = ~0u;
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt) {
         const float inv = 1.0f / fmaxf(total[32 * qt + col], 1.0e-20f);
@@ -638,9 +646,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_f32_d512_kernel(Onli
             for (int i = 0; i < 16; ++i) {
                 o[qt][dt][i] *= inv;
                 bad = __builtin_fmaf(o[qt][dt][i], 0.0f, bad);
+                smallest = min(smallest, nonzero_magnitude(o[qt][dt][i]));
             }
     }
-    if (bad != bad) atomicOr(&special, 1);
+    if (results_too_small(smallest) || bad != bad) special = 1;
     __syncthreads();
     bool redo = __builtin_amdgcn_readfirstlane(special) != 0;
     if (__builtin_expect(redo, 0))

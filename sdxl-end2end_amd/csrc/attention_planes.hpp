@@ -1,5 +1,12 @@
-// Exact splits of fp32 values into 16-bit planes and the matrix instruction
-// that multiplies them, shared by the attention kernels of fp32 accuracy.
+// Splits of fp32 values into 16-bit planes and the matrix instruction that
+// multiplies them, shared by the attention kernels of fp32 accuracy.
+//
+// Three bf16 planes hold all 24 bits of an fp32 value of at least 2^-110: below,
+// the third (then the second) falls under bf16's smallest subnormal, 2^-133
+// (the matrix cores keep subnormals), and the value is off by up to 2^-134. The
+// kernels see to it that this does not show: probabilities are scaled by 2^16;
+// a Q value below 2^-110, or so large that 2^-134 of K would count, and results
+// below 2^-100, where 2^-134 of V would, make a query block start over in fp32.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -33,6 +40,20 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 }
 __device__ __forceinline__ float lo_bf16(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
 __device__ __forceinline__ float hi_bf16(uint32_t v) { return __builtin_bit_cast(float, v & 0xFFFF0000u); }
+
+// |x| as an integer that orders like it, zero above all others.
+__device__ __forceinline__ uint32_t nonzero_magnitude(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 1u; }
+constexpr uint32_t magnitude_of_exponent(int e) { return ((uint32_t)(e + 127) << 24) - 1u; }
+
+// Whether planes give the scores of queries in full, from the smallest nonzero
+// magnitude and the largest absolute value among them: their own planes are
+// exact, and an error of 2^-134 in each of 512 values of K moves a score by less
+// than 2^-29 log2 units (c: the softmax scale in those units).
+__device__ __forceinline__ bool planes_carry_queries(uint32_t smallest, float largest, float c) {
+    return smallest >= magnitude_of_exponent(-110) && largest * fmaxf(c, 1.0f) <= 0x1p95f;
+}
+// Whether results may have lost bits of V.
+__device__ __forceinline__ bool results_too_small(uint32_t smallest) { return smallest < magnitude_of_exponent(-100); }
 
 // a less the low (kHi: high) fp16 value of h, in one instruction.
 template <bool kHi>

@@ -5,12 +5,12 @@
 // src/cuda/ops_kernels.cu:491-630, :1355-1419).
 //
 // Arithmetic: the 16-bit matrix cores run 16x the rate of the fp32 ones, so
-// fp32 operands are split exactly into three bf16 planes (8 + 8 + 8 significant
-// bits, x = h + m + l) and a product is the six plane products whose weight is
+// fp32 operands are split into three bf16 planes (8 + 8 + 8 significant bits,
+// x = h + m + l; attention_planes.hpp) and a product is the six plane products whose weight is
 // at least 2^-17 of it (hh, hm, mh, mm, hl, lh); the dropped ones weigh 2^-26,
 // below an fp32 rounding. fp16 and bf16 inputs are one plane, exact. The
 // probabilities, fp32 in the per-row kernel, keep their bits as planes too:
-// three bf16 planes for fp32 and bf16 calls, three fp16 planes scaled by 2^15
+// three bf16 planes scaled by 2^16 for fp32 and bf16 calls, three fp16 planes by 2^15
 // for fp16 calls: all 24 bits of those from 2^-16 of the row's largest on, below
 // within 2^-40 of it, which times the largest fp16 value is the smallest one
 // ([2, 8, 1000, 80] 30.1 us; two planes, 22 bits, took 27.3). All sums are fp32.
@@ -37,7 +37,7 @@
 // LDS rows are 64-dim panels of 128 bytes, 16-byte chunks XOR-swizzled by row.
 //
 // Values that planes cannot carry (infinities, NaN, fp32 above the largest
-// bf16) leave NaN in the results; a query block with any starts over in plain
+// bf16; fp32 below 2^-110 where it counts) leave NaN or tiny results; a query block with any starts over in plain
 // fp32, its rows dealt to the waves of its key groups (redo_rows).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -74,9 +74,9 @@ __device__ __forceinline__ float wave_sum(float x) {
 }
 
 template <typename T> struct Planes;
-template <> struct Planes<float> { static constexpr int in = 3, prob = 3; static constexpr bool f16 = false; static constexpr float shift = 0.0f; };
-template <> struct Planes<__bf16> { static constexpr int in = 1, prob = 3; static constexpr bool f16 = false; static constexpr float shift = 0.0f; };
-template <> struct Planes<_Float16> { static constexpr int in = 1, prob = 3; static constexpr bool f16 = true; static constexpr float shift = 15.0f; };
+template <> struct Planes<float> { static constexpr int in = 3, prob = 3; static constexpr bool f16 = false; static constexpr float weight = 65536.0f; };
+template <> struct Planes<__bf16> { static constexpr int in = 1, prob = 3; static constexpr bool f16 = false; static constexpr float weight = 65536.0f; };
+template <> struct Planes<_Float16> { static constexpr int in = 1, prob = 3; static constexpr bool f16 = true; static constexpr float weight = 32768.0f; };
 
 // Eight values of a row as loaded (fp32: two registers of four; 16-bit: one).
 template <typename T> struct Raw { u32x4 v[sizeof(T) == 4 ? 2 : 1]; };
@@ -290,6 +290,9 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
     // Q planes: lane holds query q0 + col, dims 16 ks + 8 hf .. +7.
     const int my_query = q0 + col;
     i16x8 qop[kIn][kSteps];
+    const float c = p.scale * 1.4426950408889634f;
+    uint32_t q_smallest = ~0u;
+    float q_largest = 0.0f;
     {
         const uint32_t off = (uint32_t)min(my_query - wg_q0, p.q_seq - 1 - wg_q0) * (uint32_t)(p.q_row_stride * (int64_t)sizeof(T));
         const char* src = (const char*)(qbase + (int64_t)wg_q0 * p.q_row_stride);
@@ -297,6 +300,13 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
         for (int ks = 0; ks < kSteps; ++ks) {
             const int d0 = 16 * ks + 8 * hf;
             const Raw<T> r = load8<T, kVec>(src, off, d0, D);
+            if constexpr (sizeof(T) == 4)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float x = __builtin_bit_cast(float, (uint32_t)r.v[i >> 2][i & 3]);
+                    q_smallest = min(q_smallest, nonzero_magnitude(x));
+                    q_largest = fmaxf(q_largest, fabsf(x));
+                }
             u32x4 pl[kIn];
             planes8<T>(r, pl);
             zero_past<kIn>(pl, D - d0);
@@ -304,6 +314,7 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
             for (int i = 0; i < kIn; ++i) qop[i][ks] = __builtin_bit_cast(i16x8, pl[i]);
         }
     }
+    const bool q_carried = __builtin_amdgcn_ballot_w64(!planes_carry_queries(q_smallest, q_largest, c)) == 0;
 
     // Stage loads: chunk n of the stage is row n / kChunks (sub-tile row / 32),
     // dims 8 (n % kChunks) .. +7.
@@ -368,7 +379,6 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
     float m_run = -__builtin_inff(), l_run = 0.0f;  // log2 units; this lane's half of the sum
-    const float c = p.scale * 1.4426950408889634f;
     const char* const ksub = lds + kg * (2 * kSub);
     const char* const vsub = ksub + kSub;
 
@@ -423,10 +433,10 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[t][i] *= alpha;
         }
-        const float shift = m_run == -__builtin_inff() ? 0.0f : Planes<T>::shift - m_run;
+        const float shift = m_run == -__builtin_inff() ? 0.0f : -m_run;
         f32x16 pr;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) pr[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c, shift));
+        for (int i = 0; i < 16; ++i) pr[i] = Planes<T>::weight * __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c, shift));
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(m_run) <= 1.0e6f)) != 0, 0)) {
             // no finite score yet (zero weights, as if not visible), or a
             // maximum so large that its own product with c rounds by more than
@@ -438,7 +448,7 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
                 x -= m_run;
                 // a NaN that came with no finite score must still reach the check below
                 if (m_run == -__builtin_inff() && sc[i] != sc[i]) l_run = sc[i];
-                pr[i] = m_run == -__builtin_inff() ? 0.0f : fabsf(m_run) <= 1.0e6f ? pr[i] : __builtin_amdgcn_exp2f(x + Planes<T>::shift);
+                pr[i] = m_run == -__builtin_inff() ? 0.0f : fabsf(m_run) <= 1.0e6f ? pr[i] : Planes<T>::weight * __builtin_amdgcn_exp2f(x);
             }
         }
 #pragma unroll
@@ -506,16 +516,19 @@ __global__ __launch_bounds__(256, kOcc) void tiled_attention_kernel(OnlineAttent
     const float inv = 1.0f / fmaxf(l_tot, 1.0e-20f);
     // Planes turn an infinity, a NaN or an FP32 value above the largest bf16
     // into a NaN, which reaches every score or output that it meets: a query
-    // block with one (or whose results overflow) starts over in fp32.
+    // block with one (or whose results overflow, or are so small that planes
+    // may have lost bits of them) starts over in fp32.
     float bad = l_tot;
+    uint32_t smallest = ~0u;
 #pragma unroll
     for (int t = 0; t < kTiles; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             acc[t][i] *= inv;
             bad = __builtin_fmaf(acc[t][i], 0.0f, bad);
+            if constexpr (sizeof(T) == 4) smallest = min(smallest, nonzero_magnitude(acc[t][i]));
         }
-    if (kg == 0) special[wave / kKS] = __builtin_amdgcn_ballot_w64(bad != bad) != 0;
+    if (kg == 0) special[wave / kKS] = !q_carried || __builtin_amdgcn_ballot_w64(results_too_small(smallest) || bad != bad) != 0;
     __syncthreads();  // also: nobody reads the tiles or the parked sums any more
     if (__builtin_expect(__builtin_amdgcn_readfirstlane(special[wave / kKS]) != 0, 0)) {
 #pragma unroll 1

@@ -201,3 +201,43 @@ def test_tiled_small_probabilities_keep_their_bits(D, dtype):
     bound = ref * (OUT_ROUNDING[dtype] + 2.0 ** -18) + (2.0 ** -25 + 2.0 ** -24 if dtype == "f16" else 0)
     worst = ((got - ref).abs() / bound).max().item()
     assert worst <= 1, worst
+
+
+@pytest.mark.parametrize("D,H,S", [(64, 2, 100), (72, 40, 300), (33, 2, 70), (512, 1, 100), (512, 9, 950)])
+@pytest.mark.parametrize("small", ["v", "q", "k", "weights", "one q", "part of v"])
+def test_small_fp32_values_keep_their_bits(D, H, S, small):
+    """FP32 values below 2^-110, whose third bf16 plane would fall under bf16's range, count in full: V
+    alone, Q or K against values that bring the scores back to the ordinary, weights below 2^-110 whose V
+    does, one Q value of a row, and a column of V."""
+    keys = 90
+    q, k, v = tensors(S + D, 1, H, S, keys, D, "f32")
+    tiny, huge = 2.0 ** -118, 2.0 ** 118
+    if small == "v":
+        v = v * tiny
+    elif small == "q":
+        q, k = q * tiny, k * huge
+    elif small == "k":
+        q, k = q * huge, k * tiny
+    elif small == "one q":
+        q[0, 3, 1], k[0, :, 1] = 2.0 ** -123 / 3, k[0, :, 1] * 2.0 ** 123
+        q[0, :3, 1] = q[0, 4:, 1] = 0
+    elif small == "part of v":
+        v[..., 2] *= tiny
+    else:  # one key far above the rest, whose V is zero
+        q, k = torch.zeros_like(q), torch.zeros_like(k)
+        q[..., ::D] = torch.linspace(84, 86, S, device=DEV)[None, :, None] * D ** 0.5
+        k[..., ::D] = -1
+        k[:, 7, ::D] = 0
+        v = v * 2.0 ** 100
+        v[:, 7] = v[:, 32:] = 0
+    got, ref = sh.attention(q, k, v, H).double(), reference(q, k, v, H)
+    err = (got - ref).abs()
+    if small == "part of v":  # column by column: a tiny column must be right beside ordinary ones
+        cols = torch.zeros_like(err, dtype=torch.bool)
+        cols[..., 2] = True
+        worst = max((err[cols].norm() / ref[cols].norm()).item(), (err[~cols].norm() / ref[~cols].norm()).item())
+    else:
+        rows = slice(3, 4) if small == "one q" else slice(None)
+        worst = (err[:, rows].norm() / ref[:, rows].norm()).item()
+    # fp32 sums: a few 1e-7; a fp32 argument of exp2 near 120 moves a weight by up to 2^-17
+    assert worst <= (2.0 ** -17 if small == "weights" else 2e-6), worst
