@@ -567,7 +567,7 @@ hipError_t launch_one(const OnlineAttentionParams& p, hipStream_t stream) {
     constexpr int kRows = 128 / kKS;
     const int64_t q_blocks = ((int64_t)p.q_seq + kRows - 1) / kRows;
     const int64_t grid = q_blocks * p.heads * p.batch;
-    if (grid > INT32_MAX) return hipErrorInvalidConfiguration;
+    if (grid > 0xFFFFFFFFll / 256) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((tiled_attention_kernel<T, kDp, kKS, kVec, kOcc>), dim3((unsigned)grid), dim3(256), 0, stream, p, (int)q_blocks);
     return hipGetLastError();
 }
@@ -619,7 +619,11 @@ hipError_t launch_type(const OnlineAttentionParams& p, int compute_units, hipStr
 bool tiled_attention_eligible(const OnlineAttentionParams& p, int dtype) {
     // 32-bit row offsets within a stage of at most 128 rows
     const int64_t limit = int64_t{1} << 23;
-    return dtype >= 0 && dtype <= 2 && p.head_dim <= 160 && p.k_seq > 0 && p.q_row_stride < limit && p.k_row_stride < limit &&
+    // a grid dimension holds fewer than 2^32 threads (large grids take 64
+    // queries per workgroup or more); the per-row kernel's workgroups of four
+    // rows fit more batches and heads of one row each
+    const int64_t workgroups = ((int64_t)p.q_seq + 63) / 64 * p.heads * p.batch;
+    return workgroups <= 0xFFFFFFFFll / 256 && dtype >= 0 && dtype <= 2 && p.head_dim <= 160 && p.k_seq > 0 && p.q_row_stride < limit && p.k_row_stride < limit &&
            p.v_row_stride < limit;
 }
 

@@ -241,3 +241,12 @@ def test_small_fp32_values_keep_their_bits(D, H, S, small):
         worst = (err[:, rows].norm() / ref[:, rows].norm()).item()
     # fp32 sums: a few 1e-7; a fp32 argument of exp2 near 120 moves a weight by up to 2^-17
     assert worst <= (2.0 ** -17 if small == "weights" else 2e-6), worst
+
+
+def test_more_heads_than_a_grid_of_tiles_holds():
+    """2^24 + 256 single-row (batch, head) pairs: more workgroups of tiles than a launch takes, a quarter as
+    many on the per-row kernel. One key: the output is V."""
+    B, H, D = 2 ** 19 + 8, 32, 8
+    q = torch.ones(B, 1, H * D, device=DEV, dtype=torch.float16)
+    v = torch.randn(B, 1, H * D, device=DEV, dtype=torch.float16)
+    assert torch.equal(sh.attention(q, q, v, H), v)
