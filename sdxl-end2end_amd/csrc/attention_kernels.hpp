@@ -77,7 +77,8 @@ hipError_t launch_online_attention(const OnlineAttentionParams& params, int dtyp
 
 // Tiled attention on the 16-bit matrix cores with operands and probabilities as
 // 16-bit planes (fp32 accuracy): every dtype, head_dim <= 160, key masks, causal.
-bool tiled_attention_eligible(const OnlineAttentionParams& params, int dtype);
+// compute_units as for launch_fused_attention_d64 (few queries against few keys stay on the per-row kernel).
+bool tiled_attention_eligible(const OnlineAttentionParams& params, int dtype, int compute_units);
 hipError_t launch_tiled_attention(const OnlineAttentionParams& params, int dtype, int compute_units, hipStream_t stream);
 
 // FP32 head_dim 512 on split bf16 planes (the VAE mid-block attention):

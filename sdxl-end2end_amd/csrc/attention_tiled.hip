@@ -616,15 +616,34 @@ hipError_t launch_type(const OnlineAttentionParams& p, int compute_units, hipStr
 
 }  // namespace
 
-bool tiled_attention_eligible(const OnlineAttentionParams& p, int dtype) {
+// Few queries against few keys leave most of a 64-query tile empty: with at
+// least eight (batch, head) pairs per CU the per-row kernel is the faster one as
+// long as it has few keys in all to walk per pair, a row counting as six more.
+// Measured, tiled against per-row kernel, 2048 pairs, FP32 (line at 90): 1 x 40
+// head_dim 40 28.7 / 21.6 us, 160 115 / 52; 4 x 16 20.6 / 19.1, 82 / 55; 1 x 77 41
+// / 44, 149 / 99; 4 x 40 29.5 / 47.5, 117 / 108; 16 x 4 21 / 36, 84 / 86; fp16 (line at 40): 1 x 16
+// 11.7 / 9.0, 23.9 / 15.6; 4 x 4 11.6 / 10.6, 24.0 / 16.4; 1 x 40 16.2 / 15.9, 33 /
+// 43. FP32 calls of at most four keys also on grids that the per-row kernel
+// fills only once (4 x 4, 512 pairs 8.1 / 5.8 and 20.6 / 8.8; 16 pairs 6.2 / 5.5 and
+// 10.6 / 7.8).
+static bool few_enough_for_rows(const OnlineAttentionParams& p, bool fp32, int compute_units) {
+    const int64_t cus = compute_units > 0 ? compute_units : 256;
+    const int64_t pairs = (int64_t)p.heads * p.batch, rows = pairs * p.q_seq;
+    if (rows >= int64_t{1} << 26) return false;  // more workgroups of four rows than a grid holds
+    if (pairs >= 8 * cus && (int64_t)p.q_seq * ((int64_t)p.k_seq + 6) <= (fp32 ? 90 : 40)) return true;
+    return fp32 && p.k_seq <= 4 && rows <= 8 * cus;
+}
+
+bool tiled_attention_eligible(const OnlineAttentionParams& p, int dtype, int compute_units) {
+    if (few_enough_for_rows(p, dtype == 2, compute_units)) return false;
     // 32-bit row offsets within a stage of at most 128 rows
     const int64_t limit = int64_t{1} << 23;
     // a grid dimension holds fewer than 2^32 threads (large grids take 64
     // queries per workgroup or more); the per-row kernel's workgroups of four
     // rows fit more batches and heads of one row each
     const int64_t workgroups = ((int64_t)p.q_seq + 63) / 64 * p.heads * p.batch;
-    return workgroups <= 0xFFFFFFFFll / 256 && dtype >= 0 && dtype <= 2 && p.head_dim <= 160 && p.k_seq > 0 && p.q_row_stride < limit && p.k_row_stride < limit &&
-           p.v_row_stride < limit;
+    return workgroups <= 0xFFFFFFFFll / 256 && dtype >= 0 && dtype <= 2 && p.head_dim <= 160 && p.k_seq > 0 &&
+           p.q_row_stride < limit && p.k_row_stride < limit && p.v_row_stride < limit;
 }
 
 hipError_t launch_tiled_attention(const OnlineAttentionParams& p, int dtype, int compute_units, hipStream_t stream) {

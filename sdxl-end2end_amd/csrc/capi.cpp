@@ -203,7 +203,7 @@ sdxl_status sdxl_attn_fwd(const sdxl_attn_desc* d, const void* q, const void* k,
 
     // The fused kernels form exp2 arguments as c * S and shift raw scores by
     // m / c (c = scale * log2 e); a scale so small that 1 / c overflows runs
-    // on the per-row kernel, which multiplies by the scale directly.
+    // on the kernels that multiply by the scale directly (tiled or per-row).
     const float scale_log2 = scale * 1.4426950408889634f;
     if (backend != SDXL_ATTN_WARP_ONLINE && !std::isfinite(1.0f / scale_log2)) backend = SDXL_ATTN_WARP_ONLINE;
 
@@ -221,10 +221,11 @@ sdxl_status sdxl_attn_fwd(const sdxl_attn_desc* d, const void* q, const void* k,
         // FP32 at head_dim 512 (the VAE's attention) runs on the bf16 matrix
         // cores when the call allows (auto backend, no mask, non-causal,
         // aligned rows), head_dim <= 160 on the tiled kernel; an explicit
-        // warp-online request keeps the per-row kernel.
+        // warp-online request and calls of few queries and keys keep the
+        // per-row kernel.
         if (d->backend == SDXL_ATTN_AUTO && sdxl_hip::attention_f32_d512_eligible(p, d->dtype))
             err = sdxl_hip::launch_attention_f32_d512(p, compute_units(), s);
-        else if (d->backend == SDXL_ATTN_AUTO && sdxl_hip::tiled_attention_eligible(p, d->dtype))
+        else if (d->backend == SDXL_ATTN_AUTO && sdxl_hip::tiled_attention_eligible(p, d->dtype, compute_units()))
             err = sdxl_hip::launch_tiled_attention(p, d->dtype, compute_units(), s);
         else err = sdxl_hip::launch_online_attention(p, d->dtype, s);
     } else {

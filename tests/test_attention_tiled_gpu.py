@@ -250,3 +250,17 @@ def test_more_heads_than_a_grid_of_tiles_holds():
     q = torch.ones(B, 1, H * D, device=DEV, dtype=torch.float16)
     v = torch.randn(B, 1, H * D, device=DEV, dtype=torch.float16)
     assert torch.equal(sh.attention(q, q, v, H), v)
+
+
+@pytest.mark.parametrize("dtype,B,H,Sq,Sk,D", [
+    ("f32", 256, 8, 1, 84, 40), ("f32", 128, 16, 4, 16, 160), ("f32", 1, 8, 3, 4, 80), ("f32", 32, 64, 1, 1, 7),
+    ("f16", 256, 8, 1, 34, 80), ("bf16", 256, 8, 4, 4, 40)])
+def test_few_queries_and_keys_on_the_per_row_kernel(dtype, B, H, Sq, Sk, D):
+    """Calls on whose tiles most queries would be missing take the per-row kernel: its results, bit for bit,
+    with a key mask and a causal limit too."""
+    q, k, v = tensors(Sk, B, H, Sq, Sk, D, dtype)
+    mask = (torch.rand(B, Sk, device=DEV, generator=torch.Generator(device=DEV).manual_seed(3)) < 0.7).int()
+    for causal in (False, True):
+        for key_mask in (None, mask):
+            assert torch.equal(sh.attention(q, k, v, H, causal=causal, key_mask=key_mask),
+                               sh.attention(q, k, v, H, causal=causal, key_mask=key_mask, backend=sh.WARP_ONLINE))
