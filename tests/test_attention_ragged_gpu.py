@@ -114,3 +114,34 @@ def test_masked_largest_weight_is_exact(B, H, S, top, causal, dtype):
     half_unit = torch.exp2(torch.floor(torch.log2(ref))) * UNIT[dtype]
     excess = ((got.double() - ref).abs() - half_unit) / ref
     assert excess.max().item() <= 2.0 ** -17, excess.max().item()
+
+
+# as in test_ragged: key-split workgroups on either kernel, mixed ones within one head and across two, whole ones
+KINDS = [(1, 2, 450, 449), (1, 75, 700, 450), (2, 16, 2560, 129), (4, 20, 930, 223), (2, 20, 300, 300)]
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("B,H,Sq,Sk", KINDS)
+@pytest.mark.parametrize("masked", [False, True])
+def test_ragged_strided_rows(B, H, Sq, Sk, masked, dtype):
+    """K and V as column slices of one wide buffer (equal strides), and K from a wider buffer than V, with
+    which a mixed workgroup stays within one head."""
+    W = H * 64
+    g = torch.Generator(device=DEV).manual_seed(Sk)
+    wide = torch.randn(B, Sk, 3 * W + 64, device=DEV, generator=g).to(DTYPES[dtype])
+    q = torch.randn(B, Sq, W, device=DEV, generator=g).to(DTYPES[dtype])
+    v = torch.randn(B, Sk, W + 8, device=DEV, generator=g).to(DTYPES[dtype])
+    mask = torch.ones(B, Sk, dtype=torch.int32, device=DEV)
+    mask[:, Sk // 3: Sk // 2] = 0
+    for key, value in ((wide[..., W:2 * W], wide[..., 2 * W:3 * W]), (wide[..., 8:W + 8], v[..., :W])):
+        check(q, key, value, H, dtype, key_mask=mask if masked else None)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 2, 450, 449), (1, 75, 700, 450), (1, 32, 2560, 129), (1, 80, 930, 223),
+                                       (1, 40, 300, 300)])
+def test_ragged_rows_past_the_keys_are_not_read_into_the_result(B, H, Sq, Sk):
+    """K and V are the leading rows of longer buffers whose next rows are NaN."""
+    q, k, v = tensors(Sk, B, H, Sq, Sk + 128, "f16")
+    k[:, Sk:] = v[:, Sk:] = float("nan")
+    check(q, k[:, :Sk], v[:, :Sk], H, "f16")
+    check(q, k[:, :Sk], v[:, :Sk], H, "f16", causal=True)

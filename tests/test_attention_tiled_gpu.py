@@ -264,3 +264,29 @@ def test_few_queries_and_keys_on_the_per_row_kernel(dtype, B, H, Sq, Sk, D):
         for key_mask in (None, mask):
             assert torch.equal(sh.attention(q, k, v, H, causal=causal, key_mask=key_mask),
                                sh.attention(q, k, v, H, causal=causal, key_mask=key_mask, backend=sh.WARP_ONLINE))
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("D", [80, 128, 160, 90, 127])  # aligned rows, and rows that are not at padded 96 and 128
+def test_tiled_two_key_groups(D, dtype):
+    """512 blocks of 32 queries: two key groups at every padded head dimension above 64, in 16 bits too."""
+    q, k, v = tensors(D, 2, 8, 1000, 150, D, dtype)
+    for causal in (False, True):
+        check(sh.attention(q, k, v, 8, causal=causal), reference(q, k, v, 8, causal), dtype)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 9, 950, 32), (1, 9, 950, 33), (1, 9, 950, 64), (1, 6, 1000, 31)])
+def test_d512_few_key_blocks(B, H, Sq, Sk):
+    """64 queries per workgroup with one key block, one and a bit, and two; 32 queries with less than one."""
+    q, k, v = tensors(Sq + Sk, B, H, Sq, Sk, 512, "f32")
+    check(sh.attention(q, k, v, H), reference(q, k, v, H), "f32")
+
+
+@pytest.mark.parametrize("H,Sq,Sk,D", [(1, 70, 45, 512), (9, 950, 45, 512), (6, 1000, 70, 512), (1, 40, 31, 512),
+                                       (2, 100, 77, 64), (8, 2000, 150, 80), (2, 70, 45, 33)])
+def test_rows_past_the_keys_are_not_read_into_the_result(H, Sq, Sk, D):
+    """K and V are the leading rows of longer buffers whose next rows are NaN."""
+    q, k, v = tensors(Sq + Sk, 1, H, Sq, Sk + 64, D, "f32")
+    k[:, Sk:] = v[:, Sk:] = float("nan")
+    k, v = k[:, :Sk], v[:, :Sk]
+    check(sh.attention(q, k, v, H), reference(q, k, v, H), "f32")
