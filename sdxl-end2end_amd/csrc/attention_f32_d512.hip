@@ -38,7 +38,7 @@
 // instructions and the exchange of the partials (MFMA 3072 of ~6800 cycles).
 // Measured against fp32 matrix instructions (v_mfma_f32_32x32x2, the same
 // outputs within 64-bit error 2.0e-6 here, 2.3e-6 there): 16384 tokens 5.02 ->
-// 2.64 ms (208 TFLOP/s), 8192 1.43 -> 0.90, 4096 0.403 -> 0.353 (two
+// 2.65 ms (208 TFLOP/s), 8192 1.43 -> 0.86, 4096 0.403 -> 0.342 (two
 // workgroups per block; one: 0.400), 1024 105 -> 83 us. Tried and not kept:
 // the residuals x - h by v_dot2 (fewer instructions, but wait states: 2.92
 // ms), K loads of 64-byte row segments exchanged by v_permlane16_swap (4096
@@ -694,7 +694,7 @@ bool attention_f32_d512_eligible(const OnlineAttentionParams& p, int dtype) {
 hipError_t launch_attention_f32_d512(const OnlineAttentionParams& p, int compute_units, hipStream_t stream) {
     if (p.batch == 0 || p.q_seq == 0) return hipSuccess;
     // One workgroup per CU at a time. 64 queries per workgroup take 1.65x the
-    // time of 32 per key block (16384 tokens: 2.59 ms against 3.1 in two rounds
+    // time of 32 per key block (16384 tokens: 2.6 ms against 3.1 in two rounds
     // of 32); with at most half the CUs' worth of 32-query blocks, two
     // workgroups share a block's output dims (each forms all of its scores).
     const int64_t heads_total = (int64_t)p.heads * p.batch;

@@ -199,7 +199,7 @@ static_assert(2 * 34 * 64 * 4 + (kMixedFull + 2) * 32 * kRowBytes <= 2 * (kKRing
 constexpr int kPlain = 0, kFirst = 1, kHide = 2, kLast = 3;
 
 // The kernel body for one workgroup kind. kTail: k_seq need not fill the last
-// tile or stage (key-split and mixed kinds; the whole kind always handles it).
+// tile or stage (masked calls, kMaskAll, always handle that).
 template <int kWaves, bool IsBf16, bool kMaskAll, int kKind, bool kTail>
 __device__ __attribute__((always_inline)) inline void attention_body(const FusedAttentionParams& p,
                                                                      char (*ring)[kTileBytes]) {
@@ -456,7 +456,8 @@ __device__ __attribute__((always_inline)) inline void attention_body(const Fused
     // issue of a transfer holds its wave for tens of cycles, and whole waves
     // then issue one instead of two (c3 90.9 -> 88.2 us; moving V to the half
     // waves as well measured no faster). Every wave's slabs have parity w & 1,
-    // one per-lane offset per wave; k_seq % 64 == 0. The head index is a
+    // one per-lane offset per wave; a tile that k_seq does not fill (kTail) goes
+    // slab by slab through tail_slab. The head index is a
     // compile-time loop variable so the base pointers stay scalars.
     const char* set_k0 = (const char*)p.k + ((int64_t)(bh_set[0] / p.heads) * p.k_seq * p.k_row_stride +
                                              (int64_t)(bh_set[0] % p.heads) * kHeadDim) * elem;

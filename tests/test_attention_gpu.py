@@ -232,10 +232,10 @@ def test_fp32_vae_head_dim_512():
 
 
 # ---------------------------------------------------------------- FP32, head_dim 512 (VAE)
-# The VAE mid-block's single-head FP32 attention (src/cuda/vae.cpp:89-92) runs on the fp32
-# matrix cores when unmasked and non-causal: 64-, 32- or 16-query workgroups (by how many fill the
-# CUs), 32-key blocks, ragged tails. The small shapes run 16-query workgroups; Sq 8192 (one head)
-# 32-query ones, Sq 16384 64-query ones.
+# The VAE mid-block's single-head FP32 attention (src/cuda/vae.cpp:89-92) runs on split bf16 planes
+# when unmasked and non-causal: 64- or 32-query workgroups (by the rounds they make on the CUs), two
+# workgroups per 32-query block on small grids, 32-key blocks, ragged tails. The small shapes run two
+# workgroups per block; Sq 8192 (one head) 32-query ones, Sq 16384 64-query ones.
 
 @pytest.mark.parametrize("B,Sq,Sk,H", [
     (1, 1, 1, 1), (1, 33, 1, 1), (1, 64, 64, 1), (1, 100, 77, 1), (2, 257, 300, 1),
@@ -263,8 +263,8 @@ def test_fp32_d512_strided_rows():
 @pytest.mark.parametrize("B,H", [(1, 1), (2, 1), (2, 2)])
 def test_fp32_d512_vae_latent_64x64(B, H):
     """4096 tokens (a 512x512 image's VAE mid-block) against a float64 torch reference on the
-    device; (1, 1) runs 16-query workgroups, (2, 1) 32-query ones, (2, 2) fills the CUs with
-    64-query workgroups."""
+    device; (1, 1) runs two workgroups per 32-query block, (2, 1) one, (2, 2) 64-query
+    workgroups."""
     g = torch.Generator(device=DEV)
     g.manual_seed(775)
     q, k, v = (torch.randn(B, 4096, H * 512, device=DEV, generator=g) for _ in range(3))
