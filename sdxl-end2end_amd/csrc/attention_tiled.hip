@@ -638,9 +638,8 @@ bool tiled_attention_eligible(const OnlineAttentionParams& p, int dtype, int com
     if (few_enough_for_rows(p, dtype == 2, compute_units)) return false;
     // 32-bit row offsets within a stage of at most 128 rows
     const int64_t limit = int64_t{1} << 23;
-    // a grid dimension holds fewer than 2^32 threads (large grids take 64
-    // queries per workgroup or more); the per-row kernel's workgroups of four
-    // rows fit more batches and heads of one row each
+    // a grid dimension holds fewer than 2^32 threads (the caller splits batches;
+    // large grids take 64 queries per workgroup or more)
     const int64_t workgroups = ((int64_t)p.q_seq + 63) / 64 * p.heads * p.batch;
     return workgroups <= 0xFFFFFFFFll / 256 && dtype >= 0 && dtype <= 2 && p.head_dim <= 160 && p.k_seq > 0 &&
            p.q_row_stride < limit && p.k_row_stride < limit && p.v_row_stride < limit;

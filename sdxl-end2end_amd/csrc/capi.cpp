@@ -6,6 +6,7 @@
 // stream-ordered kernel launch. No allocation and no host synchronisation.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cctype>
 #include <cmath>
@@ -207,6 +208,31 @@ sdxl_status sdxl_attn_fwd(const sdxl_attn_desc* d, const void* q, const void* k,
     const float scale_log2 = scale * 1.4426950408889634f;
     if (backend != SDXL_ATTN_WARP_ONLINE && !std::isfinite(1.0f / scale_log2)) backend = SDXL_ATTN_WARP_ONLINE;
 
+    if (backend != SDXL_ATTN_WARP_ONLINE) {
+        const int64_t rows = sdxl_hip::fused_attention_block_queries();
+        if ((d->q_seq + rows - 1) / rows * d->heads * d->batch > INT32_MAX)
+            return fail(SDXL_STATUS_INVALID_SHAPE, "sdxl_attn: grid too large");
+    }
+    // A grid dimension holds fewer than 2^32 threads, and a launch beyond that
+    // leaves outputs unwritten without an error. Every kernel here has at most
+    // 1024 threads per 16 rows of a (batch, head) pair: longer batches go in parts.
+    const int64_t part_batch = std::max<int64_t>(1, ((int64_t{1} << 22) - 1) / (d->heads * ((d->q_seq + 15) / 16)));
+    if (d->batch > part_batch) {
+        const int64_t elem = d->dtype == SDXL_DTYPE_F32 ? 4 : 2;
+        auto at = [&](const void* base, int64_t b, int64_t seq, int64_t stride) {
+            return base == nullptr ? nullptr : (void*)((char*)const_cast<void*>(base) + b * seq * eff_stride(stride, width) * elem);
+        };
+        for (int64_t b = 0; b < d->batch; b += part_batch) {
+            sdxl_attn_desc part = *d;
+            part.batch = std::min(part_batch, d->batch - b);
+            st = sdxl_attn_fwd(&part, at(q, b, d->q_seq, d->q_row_stride), at(k, b, d->k_seq, d->k_row_stride),
+                               at(v, b, d->k_seq, d->v_row_stride), key_mask != nullptr ? key_mask + b * d->k_seq : nullptr,
+                               at(o, b, d->q_seq, d->o_row_stride), stream);
+            if (st != SDXL_STATUS_OK) return st;
+        }
+        return SDXL_STATUS_OK;
+    }
+
     hipError_t err;
     if (backend == SDXL_ATTN_WARP_ONLINE) {
         sdxl_hip::OnlineAttentionParams p{};
@@ -239,9 +265,6 @@ sdxl_status sdxl_attn_fwd(const sdxl_attn_desc* d, const void* q, const void* k,
         p.heads = (int32_t)d->heads; p.causal = d->causal != 0;
         p.scale_log2 = scale_log2;
         p.inv_scale_log2 = 1.0f / scale_log2;
-        const int64_t blocks = ((d->q_seq + sdxl_hip::fused_attention_block_queries() - 1) /
-                                sdxl_hip::fused_attention_block_queries()) * d->heads * d->batch;
-        if (blocks > INT32_MAX) return fail(SDXL_STATUS_INVALID_SHAPE, "sdxl_attn: grid too large");
         err = sdxl_hip::launch_fused_attention_d64(p, d->dtype == SDXL_DTYPE_BF16, compute_units(), s);
     }
     if (err != hipSuccess)

@@ -243,13 +243,22 @@ def test_small_fp32_values_keep_their_bits(D, H, S, small):
     assert worst <= (2.0 ** -17 if small == "weights" else 2e-6), worst
 
 
-def test_more_heads_than_a_grid_of_tiles_holds():
-    """2^24 + 256 single-row (batch, head) pairs: more workgroups of tiles than a launch takes, a quarter as
-    many on the per-row kernel. One key: the output is V."""
-    B, H, D = 2 ** 19 + 8, 32, 8
+@pytest.mark.parametrize("B,D,backend", [(2 ** 19 + 8, 8, sh.AUTO),           # tiled or per-row: 2^24 + 256 pairs
+                                         (2 ** 21 + 4, 8, sh.WARP_ONLINE),    # per-row: 2^26 + 128
+                                         (2 ** 19 + 8, 64, sh.AUTO)])         # 16-bit head_dim 64
+def test_more_pairs_than_one_grid_holds(B, D, backend):
+    """More single-row (batch, head) pairs than one launch of the kernel takes. One visible key: the output
+    is V, where a key mask leaves it."""
+    H = 32
     q = torch.ones(B, 1, H * D, device=DEV, dtype=torch.float16)
     v = torch.randn(B, 1, H * D, device=DEV, dtype=torch.float16)
-    assert torch.equal(sh.attention(q, q, v, H), v)
+    got = torch.full_like(v, float("nan"))
+    sh.attention(q, q, v, H, backend=backend, out=got)
+    assert torch.equal(got, v)
+    mask = torch.ones(B, 1, dtype=torch.int32, device=DEV)
+    mask[-1] = mask[1] = 0
+    v[-1] = v[1] = 0
+    assert torch.equal(sh.attention(q, q, v, H, key_mask=mask, backend=backend), v)
 
 
 @pytest.mark.parametrize("dtype,B,H,Sq,Sk,D", [
