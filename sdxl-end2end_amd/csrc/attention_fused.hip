@@ -1713,6 +1713,12 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
     p.whole_units = p.total_blocks;
     p.split_units = 0;
     bool wide = false;  // whole + split2 workgroups on the 64-KiB kernel
+    // Its halves are whole 64-key groups: an odd number of them leaves a wave
+    // half of its last stage empty. The 32-KiB kernel's 32-key groups divide
+    // such lengths evenly ([1, 10, 1024 x 576] 8.3 us, 10.9 on the 64-KiB kernel;
+    // [2, 20, 1024 x 1984] 28.4 / 31.9); lengths that end inside a group are
+    // uneven on either.
+    const bool wide_keys = p.k_seq % 64 != 0 || p.k_seq % 128 == 0;
     const int64_t slots = (int64_t)compute_units * 3;
     const int64_t units = p.total_blocks;
     const bool mask_all = p.causal || p.key_mask != nullptr;
@@ -1732,7 +1738,7 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
             p.split_units = (int32_t)(2 * r);
             // one round of at most two workgroups per CU: key-split workgroups
             // with 64 keys of each half per stage
-            wide = full == 0 && q == 1 && 2 * r <= compute_units;
+            wide = wide_keys && full == 0 && q == 1 && 2 * r <= compute_units;
         } else if (2 * rem >= slots) {
             p.whole_units = (int32_t)(full + 2 * rem - slots);
             p.split_units = (int32_t)(2 * slots - 2 * rem);
@@ -1741,7 +1747,7 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
             p.split_units = (int32_t)(2 * rem);
             // one round of at most two key-split workgroups per CU: the 64-KiB
             // kind too ([1,10,1024,1024] 11.5 -> 10.9 us)
-            wide = full == 0 && rem <= compute_units;
+            wide = wide_keys && full == 0 && rem <= compute_units;
         }
     }
     // Ragged calls (their last stage holds hidden keys, and a unit may hold 64
@@ -1765,7 +1771,7 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
     // the 4-wave grids in one process: [2,10,4096] 92.5 vs 94.0 us (exact
     // fit), [4,20,960] 26.5 vs 29.5 us (240 of 256 CUs busy), [4,10,3840]
     // 157.9 vs 169.9 us (two rounds, 480 workgroups).
-    const bool tail64 = p.k_seq % 64 != 0, tail128 = p.k_seq % 128 != 0;
+    const bool tail64 = p.k_seq % 64 != 0;
     if (compute_units > 0 && !mask_all && p.k_seq > 0) {
         const int64_t qb32 = (p.q_seq + 31) / 32;
         const int64_t total = qb32 * p.heads * p.batch;
@@ -1815,9 +1821,9 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
         if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, true, true, false>), grid, block, 0, stream, p);
         else hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, false, true, false>), grid, block, 0, stream, p);
     } else if (wide) {
-        if (is_bf16 && tail128) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<true, true>), grid, block, 0, stream, p);
+        if (is_bf16 && tail64) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<true, true>), grid, block, 0, stream, p);
         else if (is_bf16) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<true, false>), grid, block, 0, stream, p);
-        else if (tail128) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<false, true>), grid, block, 0, stream, p);
+        else if (tail64) hipLaunchKernelGGL((fused_attention_d64_wide_kernel<false, true>), grid, block, 0, stream, p);
         else hipLaunchKernelGGL((fused_attention_d64_wide_kernel<false, false>), grid, block, 0, stream, p);
     } else {
         if (is_bf16 && tail64) hipLaunchKernelGGL((fused_attention_d64_kernel<kFusedWaves, true, false, true>), grid, block, 0, stream, p);
