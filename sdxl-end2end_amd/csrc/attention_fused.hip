@@ -1777,7 +1777,12 @@ hipError_t launch_fused_attention_d64(const FusedAttentionParams& params_in, boo
         const int64_t total = qb32 * p.heads * p.batch;
         const int64_t wgs = (total + kMixedBlocks - 1) / kMixedBlocks;
         const int64_t rounds = (wgs + compute_units - 1) / compute_units;
-        if (qb32 >= kMixedBlocks && wgs <= INT32_MAX &&
+        // Ragged calls: two rounds only with many keys, more not, as the first and last
+        // tiles, at one workgroup per CU, are not hidden by another workgroup's
+        // ([6, 20, 4480 x 224] 65.8 us on whole workgroups, 79.0 mixed; [4, 10, 4000] x
+        // 400 29.5 / 29.9, x 1000 53.4 / 53.1; one round: [4, 20, 930 x 224] 13.7 / 12.0).
+        const bool ragged_ok = !tail64 || rounds == 1 || (rounds == 2 && p.k_seq >= 800);
+        if (ragged_ok && qb32 >= kMixedBlocks && wgs <= INT32_MAX &&
             (double)(rounds * kMixedBlocks) <= 1.10 * (double)total / (double)compute_units) {
             p.q_blocks = (int32_t)qb32;
             p.mixed_total = (int32_t)total;
