@@ -50,8 +50,8 @@ typedef enum sdxl_dtype {
  *     correctness fallback, any head_dim <= 1024, f16/bf16/f32);
  *   AUTO picks the fused kernel whenever it is eligible, else WARP_ONLINE,
  *     whose calls run tiled matrix-core kernels of fp32 accuracy instead of
- *     the per-row one where they take the shape (head_dim <= 160; unmasked
- *     non-causal FP32 at head_dim 512, the VAE). */
+ *     the per-row one where they take the shape (head_dim <= 160, more than a
+ *     few queries or keys; unmasked non-causal FP32 at head_dim 512, the VAE). */
 typedef enum sdxl_attn_backend {
     SDXL_ATTN_AUTO = 0,
     SDXL_ATTN_CUDNN_SDPA = 1,
