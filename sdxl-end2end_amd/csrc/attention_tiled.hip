@@ -211,7 +211,6 @@ __device__ __forceinline__ void redo_rows(const T* q, const T* k, const T* v, T*
             for (int t = 0; t < kChannels; ++t) acc[r][t] *= alpha;
         }
         const int n = min(64, n_keys - k0);
-#pragma unroll 4
         for (int j = 0; j < n; ++j) {
             const T* vrow = v + (int64_t)(k0 + j) * v_stride;
             float x[kChannels];
